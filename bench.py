@@ -289,6 +289,10 @@ def main():
     wall = t1 - t0
     nf = case.info.num_fluid
     n_bulk, steps_per_launch, kname = timed_kernel(s, case)
+    lds = s.lds_steps > 0
+    sampled = timed_launches(args.steps, args.sample_every, steps_per_launch, lds)
+    if lds and sampled:
+        steps_per_launch = round(sum(sampled) / len(sampled), 4)
     two = s.two_step_info()
     three = s.three_step_info()
     mlups = nf * args.steps / wall / 1e6
@@ -309,7 +313,7 @@ def main():
     if default_shape and os.path.exists(PMC_SUMMARY):
         try:
             pm = json.load(open(PMC_SUMMARY))
-            prefix = {1: "", 2: "two_", 3: "three_"}[steps_per_launch]
+            prefix = "lds_" if lds else {1: "", 2: "two_", 3: "three_"}[steps_per_launch]
             key = f"{prefix}{args.collision}_{args.precision}_{N}"
             if key in pm.get("kernels", {}):
                 traffic = pm["kernels"][key]["hbm_bytes_per_launch"]
@@ -330,6 +334,8 @@ def main():
         o64.precision = lbm.PREC_F64
         s64 = lbm.Solver(case, o64)
         n64, spl64, _ = timed_kernel(s64, case)
+        made = timed_launches(args.steps, args.sample_every, spl64, s64.lds_steps > 0)
+        spl64 = round(sum(made) / max(len(made), 1), 4) if s64.lds_steps else spl64
         s64.step(args.warmup)
         s64.sync()
         t0 = time.perf_counter()
@@ -413,7 +419,7 @@ def main():
             "state_frac": round(state_gbs / HBM_PEAK_GBS, 4),
             "traffic_over_state": round(traffic / state_bytes_per_launch, 4) if traffic else None,
             "avg_launch_us": round(avg_bulk_s * 1e6, 2),
-            "launches_timed": launches_timed(args.steps, args.sample_every, steps_per_launch),
+            "launches_timed": len(sampled),
             "copy_kernel_gbs": round(copy_gbs, 1),
             "stream_probe_gbs": round(probe_gbs, 1) if probe_gbs else None,
             "stream_probe_us": round(probe_us, 2) if probe_us else None,
@@ -424,15 +430,26 @@ def main():
     print(json.dumps(out), flush=True)
 
 
-def launches_timed(steps: int, every: int, per_launch: int) -> int:
-    """Launches lbm_solver_step_timed brackets with events in a run of plain
-    steps: those of every `every`-th step; a multi-step launch is sampled
-    when any of its steps is (a run's last steps may take a launch of fewer
-    steps, which is not sampled)."""
+def timed_launches(steps: int, every: int, per_launch: int, lds: bool) -> list[int]:
+    """Steps made by each launch lbm_solver_step_timed brackets with events in
+    a run of plain steps: those that hold every `every`-th step.  Two- and
+    three-step launches make exactly as many (a run's last steps may take a
+    launch of fewer, which is not sampled); LDS-resident ones at most
+    per_launch, the last two of a run sharing what is left, and the last step
+    of a call is a single one."""
     if per_launch == 1:
-        return (steps + every - 1) // every
-    return sum(1 for t in range(0, steps - per_launch + 1, per_launch)
-               if any((t + i) % every == 0 for i in range(per_launch)))
+        return [1] * ((steps + every - 1) // every)
+    made, t = [], 0
+    end = steps - 1 if lds else steps
+    while end - t >= (2 if lds else per_launch):
+        left = end - t
+        k = per_launch
+        if lds and left < 2 * per_launch - 1:
+            k = (left + 1) // 2 if left > per_launch else left
+        if any((t + i) % every == 0 for i in range(k)):
+            made.append(k)
+        t += k
+    return made
 
 
 def timed_kernel(s, case):
@@ -441,7 +458,11 @@ def timed_kernel(s, case):
     tiles' nodes, three steps; two-step launches: the two-step tiles' nodes,
     two steps (the band's single steps are separate launches); else the fused
     step kernel (bulk tiles and boundary-list nodes; FP16: its paired-cell
-    form) or the bulk kernel."""
+    form) or the bulk kernel.  With LDS-resident blocks, which come first, every
+    fluid node and the most steps a launch makes."""
+    if s.lds_steps:
+        return (case.info.num_fluid, s.lds_steps,
+                "k_lds_steps (runs of plain steps with LDS-resident blocks)")
     three = s.three_step_info()
     if three["cells"] > 0:
         return three["cells"], 3, "k_three_steps (three steps per launch over the three-step tiles)"
@@ -853,6 +874,9 @@ def bench_matrix(args):
                 o.precision = prec
                 s = lbm.Solver(case, o)
                 nl, spl, _ = timed_kernel(s, case)
+                if s.lds_steps:
+                    made = timed_launches(args.steps, args.sample_every, spl, True)
+                    spl = round(sum(made) / max(len(made), 1), 4)
                 s.step(args.warmup)
                 s.sync()
                 t0 = time.perf_counter()

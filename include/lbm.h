@@ -138,8 +138,13 @@ typedef struct lbm_options {
  * LBM_TUNE_NO_TILE_WALLS: every boundary node in the boundary list (by
  * default nodes whose only rule is straight-wall bounce-back run in their
  * bulk tile).
- * LBM_TUNE_NO_TWO_STEP: every step its own launch.  By default two plain
- * steps in a row run as one pass over the state where that pays (FP32
+ * LBM_TUNE_NO_TWO_STEP: every step its own launch.  By default runs of plain
+ * steps go several to a launch with each block of nodes held in LDS between
+ * them (lbm_solver_fused reports how many), on every lattice without open
+ * outlets; the last step of a call is a single one.  Captured graphs, split
+ * launches and two_step_rows or three_step_rows > 0 turn that off.
+ * Two plain steps in a row also run as one pass over the state where that
+ * pays for runs too short for the above (FP32
  * storage on lattices of at least 2^20 cells, FP64 on lattices of at least
  * 2^22 cells, two thirds of the nodes away from the boundary-list nodes; also
  * on packed lattices of instances): interior and in-tile wall
@@ -269,11 +274,12 @@ int lbm_solver_step(lbm_solver* s, int nsteps, int* done);
 /* Same, timing the step kernel with HIP events on the solver's stream around
  * every `sample_every`-th launch (1 = every launch).  total_ms: stream time of
  * the nsteps; kernel_ms: average duration of one sampled step-kernel launch.
- * With multi-step launches on (lbm_solver_two_step_info,
- * lbm_solver_three_step_info) the sampled kernel is the three-step kernel
- * (one launch per three steps) where three-step launches are on, else the
- * two-step kernel (one launch per two steps); launches of fewer steps are
- * not sampled. */
+ * With LDS-resident blocks (lbm_solver_fused) the sampled kernel is theirs,
+ * up to that many steps per launch.  With two- or three-step launches alone
+ * (lbm_solver_two_step_info, lbm_solver_three_step_info) it is the three-step
+ * kernel (one launch per three steps) where three-step launches are on, else
+ * the two-step kernel (one launch per two steps); launches of fewer steps
+ * are not sampled. */
 int lbm_solver_step_timed(lbm_solver* s, int nsteps, int sample_every, double* total_ms,
                           double* kernel_ms);
 int lbm_solver_sync(lbm_solver* s);
@@ -349,7 +355,8 @@ int lbm_solver_load(lbm_solver* s, const char* path);
  * nodes share one launch per step (else separate launches); bit 1 set if
  * plain steps run the paired-cell FP16 kernel; bit 2 set if pairs of plain
  * steps run as two-step launches; bit 3 set if runs of three plain steps run
- * as three-step launches. */
+ * as three-step launches; bits 8-15 the most plain steps that one launch with
+ * LDS-resident blocks makes (0: off). */
 int lbm_solver_fused(const lbm_solver* s);
 /* Two-step launches of this solver: *cells = nodes the two-step kernel
  * advances by two steps per launch (0: two-step launches off), *tiles = its

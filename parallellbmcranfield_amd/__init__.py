@@ -435,6 +435,11 @@ class Solver:
         """Plain steps run the paired-cell FP16 kernel."""
         return bool(lib().lbm_solver_fused(self.h) & 2)
 
+    @property
+    def lds_steps(self) -> int:
+        """The most plain steps one launch with LDS-resident blocks makes (0: off)."""
+        return lib().lbm_solver_fused(self.h) >> 8 & 0xff
+
     def two_step_info(self) -> dict:
         """Two-step launches: nodes advanced two steps per launch (0 = off),
         the kernel's tiles, and the nodes that take two single steps."""

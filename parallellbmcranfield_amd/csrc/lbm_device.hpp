@@ -87,6 +87,14 @@ struct StF64 {
 #pragma unroll
     for (int k = 0; k < 9; k++) store(plane_word(dst, kp.plane, k, idx), v[k], kp, 0u);
   }
+  static constexpr bool SCALED = false;
+  // the units of the LDS-resident steps: loads, rounding to what is stored
+  __device__ static R load_raw(const T* p) { return ld(p); }
+  __device__ static void round_raw(R (&)[9], int, uint32_t) {}
+  __device__ static void store_raw(T* dst, int idx, const R (&v)[9], const KParams& kp, uint32_t) {
+#pragma unroll
+    for (int k = 0; k < 9; k++) *plane_word(dst, kp.plane, k, idx) = v[k];
+  }
 };
 struct StF32 {
   using T = float;
@@ -100,6 +108,14 @@ struct StF32 {
   __device__ static void store_cell(T* dst, int idx, const R (&v)[9], const KParams& kp, uint32_t) {
 #pragma unroll
     for (int k = 0; k < 9; k++) store(plane_word(dst, kp.plane, k, idx), v[k], kp, 0u);
+  }
+  static constexpr bool SCALED = false;
+  // the units of the LDS-resident steps: loads, rounding to what is stored
+  __device__ static R load_raw(const T* p) { return ld(p); }
+  __device__ static void round_raw(R (&)[9], int, uint32_t) {}
+  __device__ static void store_raw(T* dst, int idx, const R (&v)[9], const KParams& kp, uint32_t) {
+#pragma unroll
+    for (int k = 0; k < 9; k++) *plane_word(dst, kp.plane, k, idx) = v[k];
   }
 };
 struct StF16 {
@@ -119,6 +135,18 @@ struct StF16 {
   __device__ static void store_cell(T* dst, int idx, const R (&v)[9], const KParams& kp, uint32_t) {
 #pragma unroll
     for (int k = 0; k < 9; k++) store(plane_word(dst, kp.plane, k, idx), v[k], kp, 0u);
+  }
+  static constexpr bool SCALED = true;
+  // the units of the LDS-resident steps: stored units, (f - w rho0) * scale
+  __device__ static R load_raw(const T* p) { return (float)ld(p); }
+  __device__ static void round_raw(R (&v)[9], int, uint32_t) {
+#pragma unroll
+    for (int k = 0; k < 9; k++) v[k] = (float)(_Float16)v[k];
+  }
+  __device__ static void store_raw(T* dst, int idx, const R (&v)[9], const KParams& kp, uint32_t) {
+#pragma unroll
+    for (int k = 0; k < 9; k++)
+      *plane_word(dst, kp.plane, k, idx) = (_Float16)v[k];
   }
 };
 
@@ -180,6 +208,21 @@ struct StF16S : StF16 {
     }
   }
   __device__ static void store_rn(T* p, R v, const KParams& kp) { StF16::store(p, v, kp, 0u); }
+  __device__ static void round_raw(R (&v)[9], int idx, uint32_t step) {
+    uint32_t r = sr_pair_bits(idx, step);
+    const bool second = (idx & 1) != 0;
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+      half2_t x = {(_Float16)0, (_Float16)0};
+      x = f16_stochastic_into(x, v[k], second ? rot16(r) : r, false);
+      v[k] = (float)x[0];
+      r = xorshift32(r);
+    }
+  }
+  __device__ static void store_raw(T* dst, int idx, R (&v)[9], const KParams& kp, uint32_t step) {
+    round_raw(v, idx, step);
+    StF16::store_raw(dst, idx, v, kp, step);  // exact: the values are FP16 ones
+  }
 };
 
 // The step number a launch stores with (stochastic-rounding storage; 0
@@ -363,8 +406,9 @@ __device__ inline void collide_trt_dev(const float g[9], float drho, float rho, 
   }
 }
 
-__device__ inline void collide_mrt_dev(const float g[9], float drho, float rho, float u, float v,
-                                       const CollPar& p, float out[9]) {
+// rs: the density in the units of g (rho itself, or scaled as g is: node_dev).
+__device__ inline void mrt_relax(const float g[9], float drho, float rho, float rs, float u,
+                                 float v, const CollPar& p, float out[9]) {
   // No implicit contraction: the fused multiply-adds are written out, so
   // every kernel that inlines this (one cell or two per thread, one step or
   // several per launch) rounds the same way.
@@ -381,16 +425,16 @@ __device__ inline void collide_mrt_dev(const float g[9], float drho, float rho, 
   const float m7 = (g[1] + g[3]) - (g[2] + g[4]);
   const float m8 = (g[5] + g[7]) - (g[6] + g[8]);
   const float usq = fmaf(u, u, v * v);
-  const float r3 = (p.flags & KF_MRT_TEXTBOOK) ? 3.f * rho * usq : 3.f * rho * rho * usq;
+  const float r3 = (p.flags & KF_MRT_TEXTBOOK) ? 3.f * rs * usq : 3.f * rho * rs * usq;
   // d_l = m_l(f) - m_l^eq; M w = (1,-2,1,0,...) absorbs rho0
   const float d1 = fmaf(2.f, drho, m1) - r3;
   const float d2 = (m2 - drho) + r3;
-  const float d3 = fmaf(-rho, u, jx);
-  const float d4 = fmaf(rho, u, m4);
-  const float d5 = fmaf(-rho, v, jy);
-  const float d6 = fmaf(rho, v, m6);
-  const float d7 = fmaf(-rho, fmaf(u, u, -(v * v)), m7);
-  const float d8 = fmaf(-rho, u * v, m8);
+  const float d3 = fmaf(-rs, u, jx);
+  const float d4 = fmaf(rs, u, m4);
+  const float d5 = fmaf(-rs, v, jy);
+  const float d6 = fmaf(rs, v, m6);
+  const float d7 = fmaf(-rs, fmaf(u, u, -(v * v)), m7);
+  const float d8 = fmaf(-rs, u * v, m8);
   // e_l = s_l d_l / |M_l|^2 ; out = g - M^T e, with the terms the columns of
   // M share formed once: columns 1-4 hold -e1 - 2 e2, columns 5-8 2 e1 + e2,
   // and the momentum / energy-flux rows enter as (e3 -+ 2 e4), (e5 -+ 2 e6)
@@ -410,6 +454,11 @@ __device__ inline void collide_mrt_dev(const float g[9], float drho, float rho, 
   out[6] = g[6] - (bm - PmQ);
   out[7] = g[7] - (bp - PQ);
   out[8] = g[8] - (bm + PmQ);
+}
+
+__device__ inline void collide_mrt_dev(const float g[9], float drho, float rho, float u, float v,
+                                       const CollPar& p, float out[9]) {
+  mrt_relax(g, drho, rho, rho, u, v, p, out);
 }
 
 template <int COLL>
@@ -453,6 +502,158 @@ __device__ inline void macro_dev(const float g[9], float rho0, float& drho, floa
   const float ir = fmaf(fmaf(-rho, ir0, 1.f), ir0, ir0);
   u = jx * ir;
   v = jy * ir;
+}
+
+// Macros and collision of one node in the deviation form with every rounding
+// written out: the fused multiply-adds are those the single-step kernels'
+// macro_dev + collide_dev compile to (k_step, MODE 0), so a kernel that uses
+// this rounds as they do however it is inlined.  The diagonal velocities
+// c.u take one component as an unrounded product: momentum times reciprocal
+// density of x (BGK, and TRT on the boundary list), of y (TRT elsewhere).
+// The terms of c.u and -c.u are formed once per direction pair.  g and out
+// are the deviations times sc, a power of two (isc its reciprocal): sc = 1, or
+// FP16 storage's fixed scale, which then needs no multiplication per load and
+// store and changes no rounding.  still: V = 0 (east outlets); list: a
+// boundary-list node.
+template <int COLL>
+__device__ inline void node_dev(const float (&g)[9], float rho0, float sc, float isc, bool still,
+                                bool list, const CollPar& p, float (&out)[9]) {
+#pragma clang fp contract(off)
+  const float drho = ((g[0] + g[1]) + (g[2] + g[3])) + ((g[4] + g[5]) + (g[6] + g[7])) + g[8];
+  const float rho = fmaf(drho, isc, rho0);
+  const float jx = (g[1] - g[3]) + (g[5] - g[7]) + (g[8] - g[6]);
+  const float jy = (g[2] - g[4]) + (g[5] - g[7]) + (g[6] - g[8]);
+  const float ir0 = __builtin_amdgcn_rcpf(rho);
+  const float ir = fmaf(fmaf(-rho, ir0, 1.f), ir0, ir0) * isc;
+  const float rs = rho * sc;  // the density in the units of g
+  const float u = jx * ir;
+  float v = jy * ir;
+  if (still) v = 0.f;
+  if constexpr (COLL == 3) {
+    mrt_relax(g, drho, rho, rs, u, v, p, out);
+  } else if constexpr (COLL == 1) {
+    const float usq = fmaf(u, u, v * v);
+    const auto put = [&](int k, float t) {
+      out[k] = fmaf(p.om, fmaf(fmaf(rs, t, drho), W32[k], -g[k]), g[k]);
+    };
+    const auto pair = [&](int k, float cu) {  // k and its opposite
+      const float q = cu * (4.5f * cu);
+      put(k, fmaf(-1.5f, usq, fmaf(3.f, cu, q)));
+      put(OPP[k], fmaf(-1.5f, usq, fmaf(-3.f, cu, q)));
+    };
+    put(0, -1.5f * usq);
+    pair(1, u);
+    pair(2, v);
+    pair(5, fmaf(jx, ir, v));
+    pair(8, fmaf(jx, ir, -v));
+  } else {
+    const float usq15 = 1.5f * fmaf(u, u, v * v);
+    const float m1 = W32[1] * rs * 3.f, m5 = W32[5] * rs * 3.f;
+    out[0] = fmaf(-p.om, fmaf(fmaf(-rs, usq15, drho), -W32[0], g[0]), g[0]);
+    const auto pair = [&](int k, float cu) {
+      const int o = OPP[k];
+      const float e = W32[k] * fmaf(rs, fmaf(cu, 4.5f * cu, -usq15), drho);
+      const float sym = fmaf(g[k] + g[o], 0.5f, -e);
+      const float asy = fmaf(g[k] - g[o], 0.5f, -((k < 5 ? m1 : m5) * cu));
+      out[k] = fmaf(-p.oma, asy, fmaf(-p.om, sym, g[k]));
+      out[o] = fmaf(p.oma, asy, fmaf(-p.om, sym, g[o]));
+    };
+    pair(1, u);
+    pair(2, v);
+    pair(5, list ? fmaf(jx, ir, v) : fmaf(jy, ir, u));
+    pair(6, list ? fmaf(-jx, ir, v) : fmaf(jy, ir, -u));
+  }
+}
+
+// macro_f64 + collide_f64 of one node with less work for the same roundings
+// in the same order, so the same values (a zero's sign aside): terms that are
+// exactly zero are left out (F times a zero component of c_k; moment 0 minus
+// its equilibrium), terms of c.u and -c.u, and products that differ in sign
+// only, are formed once, and sums with a power-of-two multiple take one fused
+// instruction (the product is exact).  still: V = 0 (east outlets).
+template <int COLL>
+__device__ inline void node_f64(const double (&F)[9], bool still, const KParams& p,
+                                double (&out)[9]) {
+  double R = F[0];
+#pragma unroll
+  for (int k = 1; k < 9; k++) R = R + F[k];
+  const double jx = F[1] - F[3] + F[5] - F[6] - F[7] + F[8];
+  const double jy = F[2] - F[4] + F[5] + F[6] - F[7] - F[8];
+  const double U = jx / R;
+  double V = jy / R;
+  if (still) V = 0.0;
+  if constexpr (COLL == 3) {
+    // collide_mrt_f64: rows 0, 3 and 5 of M F are the sums above
+    const double us = U * U + V * V;
+    const double e = 3.0 * ((p.flags & KF_MRT_TEXTBOOK) ? 1.0 : R) * us;
+    const double m1 = fma(2., F[8], fma(2., F[7], fma(2., F[6], fma(2., F[5],
+                      fma(-4., F[0], -F[1]) - F[2] - F[3] - F[4]))));
+    const double m2 = fma(-2., F[4], fma(-2., F[3], fma(-2., F[2],
+                      fma(4., F[0], -2. * F[1])))) + F[5] + F[6] + F[7] + F[8];
+    const double m4 = fma(2., F[3], -2. * F[1]) + F[5] - F[6] - F[7] + F[8];
+    const double m6 = fma(2., F[4], -2. * F[2]) + F[5] + F[6] - F[7] - F[8];
+    const double m7 = F[1] - F[2] + F[3] - F[4];
+    const double m8 = F[5] - F[6] + F[7] - F[8];
+    const double RU = R * U, RV = R * V;
+    const double d1 = m1 - R * (-2.0 + e), d2 = m2 - R * (1.0 - e), d3 = jx - RU, d4 = m4 + RU,
+                 d5 = jy - RV, d6 = m6 + RV, d7 = m7 - R * (U * U - V * V), d8 = m8 - RU * V;
+    // M^-1 S d: a column of M^-1 S holds few magnitudes
+    const double a1 = p.stmiv[0][1] * d1, b1 = p.stmiv[1][1] * d1, c1 = p.stmiv[5][1] * d1;
+    const double a2 = p.stmiv[0][2] * d2, b2 = p.stmiv[1][2] * d2, c2 = p.stmiv[5][2] * d2;
+    const double b3 = p.stmiv[1][3] * d3, b4 = p.stmiv[1][4] * d4, c4 = p.stmiv[5][4] * d4;
+    const double b5 = p.stmiv[2][5] * d5, b6 = p.stmiv[2][6] * d6, c6 = p.stmiv[5][6] * d6;
+    const double b7 = p.stmiv[1][7] * d7, c8 = p.stmiv[5][8] * d8;
+    const double b12 = b1 + b2, c12 = c1 + c2;
+    out[0] = F[0] - (a1 + a2);
+    out[1] = F[1] - (b12 + b3 + b4 + b7);
+    out[2] = F[2] - (b12 + b5 + b6 - b7);
+    out[3] = F[3] - (b12 - b3 - b4 + b7);
+    out[4] = F[4] - (b12 - b5 - b6 - b7);
+    const double cp = c12 + b3 + c4, cm = c12 - b3 - c4;
+    out[5] = F[5] - (cp + b5 + c6 + c8);
+    out[6] = F[6] - (cm + b5 + c6 - c8);
+    out[7] = F[7] - (cm - b5 - c6 + c8);
+    out[8] = F[8] - (cp - b5 - c6 - c8);
+  } else {
+    const double T15 = 1.5 * (U * U + V * V);
+    double Feq[9];
+    Feq[0] = R * W64[0] * (1.0 - T15);
+    const auto pair = [&](int k, double T2) {
+      const double a = 3.0 * T2, q = 4.5 * T2 * T2;
+      Feq[k] = R * W64[k] * (1.0 + a + q - T15);
+      Feq[OPP[k]] = R * W64[OPP[k]] * (1.0 - a + q - T15);
+    };
+    pair(1, U);
+    pair(2, V);
+    pair(5, U + V);
+    pair(6, V - U);
+    const double om = p.omega;
+    if constexpr (COLL == 1) {
+#pragma unroll
+      for (int k = 0; k < 9; k++) out[k] = om * Feq[k] + (1.0 - om) * F[k];
+    } else if (!(p.flags & KF_TRT_FP64)) {
+      out[0] = F[0] - (double)((float)F[0] - (float)Feq[0]) * om;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int k = q < 2 ? q + 1 : q + 3, o = OPP[k];
+        const float dp = (float)(0.5 * (F[k] + F[o])) - (float)(0.5 * (Feq[k] + Feq[o]));
+        const float dm = (float)(0.5 * (F[k] - F[o])) - (float)(0.5 * (Feq[k] - Feq[o]));
+        const double s = (double)dp * om, a = (double)dm * p.omega_a;
+        out[k] = F[k] - s - a;
+        out[o] = F[o] - s + a;
+      }
+    } else {
+      out[0] = F[0] - (F[0] - Feq[0]) * om;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int k = q < 2 ? q + 1 : q + 3, o = OPP[k];
+        const double s = (0.5 * (F[k] + F[o]) - 0.5 * (Feq[k] + Feq[o])) * om;
+        const double a = (0.5 * (F[k] - F[o]) - 0.5 * (Feq[k] - Feq[o])) * p.omega_a;
+        out[k] = F[k] - s - a;
+        out[o] = F[o] - s + a;
+      }
+    }
+  }
 }
 
 // ---------------------------------------------------------------- XCD-aware block order

@@ -120,6 +120,14 @@ struct lbm_solver {
   uint32_t* d_list_b3[3] = {nullptr, nullptr, nullptr};
   int nlist_b3[3] = {0, 0, 0};
   hipGraphExec_t gexec3[2] = {nullptr, nullptr};  // three-step launches by source parity
+  // several plain steps per launch with each block of nodes in LDS
+  // (k_lds_steps): every node class but open outlets
+  bool lds = false;
+  uint32_t* d_rule = nullptr;     // rule word of each padded cell (LdsRule); the two below follow
+  lbmdev::LdsList* d_lds_list = nullptr;   // rules of the boundary-list nodes
+  lbmdev::LdsTile* d_lds_tiles = nullptr;  // blocks of running instances, XCD order
+  int nlds = 0, lds_shape = 0, lds_halo = 0;
+  std::vector<lbmdev::LdsTile> lds_all;
   // the last launch was a two- or three-step one: buf[cur^1] holds the state
   // prev_lag (2 or 3) steps back, not the one step back that observe passes
   // and checkpoints read

@@ -53,27 +53,41 @@ __device__ inline double absval(typename S::R g, int k, const KParams& p) {
     return (double)g;
 }
 
+// The boundary rules of a list node, read from its record where they are used.
+struct BNodeRules {
+  const BNode& nd;
+  __device__ double uo() const { return nd.uo; }
+  __device__ bool inlet() const { return nd.boundary == 2; }
+  __device__ bool lid() const { return nd.bc[2] == 2 && nd.corner != 1; }
+  __device__ bool west() const { return nd.bc[3] == 2 && nd.corner != 1; }
+  __device__ bool wall(int k) const { return nd.bc[k] == 1; }
+  __device__ double q(int k) const { return nd.q[k]; }
+  __device__ bool east() const { return nd.bc[1] == 3; }
+};
+
 // Reference boundary rules on one node's post-streaming F (in place), in the
 // order of serial/Iterate.c:499-546: InletBC, then curved or straight walls,
 // then (profile 1) the velocity outlet.  Open outlets (profiles 2/3) are
 // applied by the caller afterwards.  R is double (absolute values) or float
 // (deviations, where every population-weighted density sum gains rho0).
-template <class S>
-__device__ inline void apply_bc(typename S::R F[9], const BNode& nd, const typename S::T* src,
-                                const KParams& p, int idx) {
+// nd gives the node's rules (BNodeRules, LdsRules); own(k) and up(k) METAF[k]
+// of the node and of its upstream neighbour in direction k.
+template <class S, class Rules, class Own, class Up>
+__device__ inline void apply_bc(typename S::R F[9], const Rules& nd, const KParams& p, Own own,
+                                Up up) {
   using R = typename S::R;
-  const R uo = (R)nd.uo;
+  const R uo = (R)nd.uo();
   const R roff = S::DEV ? (R)p.rho0 : (R)0;
   // InletBC: serial/BoundaryConditions.c:14-58
-  if (nd.boundary == 2) {
-    if (nd.bc[2] == 2 && nd.corner != 1) {
+  if (nd.inlet()) {
+    if (nd.lid()) {
       R rhoN = F[0] + F[1] + F[3] + 2 * (F[2] + F[6] + F[5]);
       if constexpr (S::DEV) rhoN = rhoN + roff;
       F[4] = F[2];
       F[8] = F[6] + rhoN * uo / (R)6.0;
       F[7] = F[5] - rhoN * uo / (R)6.0;
     }
-    if (nd.bc[3] == 2 && nd.corner != 1) {
+    if (nd.west()) {
       R num = F[0] + F[2] + F[4] + (R)2.0 * (F[3] + F[6] + F[7]);
       if constexpr (S::DEV) num = num + roff;
       const R rhoW = num / ((R)1.0 - uo);
@@ -87,15 +101,15 @@ __device__ inline void apply_bc(typename S::R F[9], const BNode& nd, const typen
     // Fneighbours[k] = METAF[k] of the upstream node (serial/Iterate.c:509-510)
 #pragma unroll
     for (int k = 0; k < 9; k++) {
-      if (nd.bc[k] == 1) {
+      if (nd.wall(k)) {
         const int o = OPP[k];
-        const R q = (R)nd.q[k];
-        const R mk = S::load(src + k * p.plane + idx, p);
-        if (nd.q[k] < 0.5) {
-          const R nk = S::load(src + k * p.plane + idx - CX[k] - CY[k] * p.pitch, p);
+        const R q = (R)nd.q(k);
+        const R mk = own(k);
+        if (nd.q(k) < 0.5) {
+          const R nk = up(k);
           F[o] = 2 * q * mk + (1 - 2 * q) * nk;
         } else {
-          const R mo = S::load(src + o * p.plane + idx, p);
+          const R mo = own(o);
           F[o] = mk / 2 / q + (2 * q - 1) / (2 * q) * mo;
         }
       }
@@ -104,9 +118,9 @@ __device__ inline void apply_bc(typename S::R F[9], const BNode& nd, const typen
     // WallBC: serial/BoundaryConditions.c:104-118 (post-streaming F[k])
 #pragma unroll
     for (int k = 0; k < 9; k++)
-      if (nd.bc[k] == 1) F[OPP[k]] = F[k];
+      if (nd.wall(k)) F[OPP[k]] = F[k];
   }
-  if (p.outlet_profile == 4 && nd.bc[1] == 3) {
+  if (p.outlet_profile == 4 && nd.east()) {
     // East pressure outlet, Zou & He (1997): rho = rho_out, v = 0; unknown
     // populations 3, 6, 7 from mass and momentum balance.
     const R ro = S::DEV ? (R)p.rho_out_f : (R)p.rho_out;
@@ -119,7 +133,7 @@ __device__ inline void apply_bc(typename S::R F[9], const BNode& nd, const typen
     F[7] = F[5] + h - t;
     F[6] = F[8] - h - t;
   }
-  if (p.outlet_profile == 1 && nd.bc[1] == 3) {
+  if (p.outlet_profile == 1 && nd.east()) {
     // OutletBoundaries: serial/BoundaryConditions.c:67-81
     R num = F[0] + F[2] + F[4] + (R)2.0 * (F[1] + F[5] + F[8]);
     if constexpr (S::DEV) num = num + roff;
@@ -128,6 +142,15 @@ __device__ inline void apply_bc(typename S::R F[9], const BNode& nd, const typen
     F[7] = F[5] - rhoE * uo / (R)6.0;
     F[6] = F[8] - rhoE * uo / (R)6.0;
   }
+}
+
+// apply_bc with the METAF values read from the state buffer src.
+template <class S>
+__device__ inline void apply_bc(typename S::R F[9], const BNode& nd, const typename S::T* src,
+                                const KParams& p, int idx) {
+  apply_bc<S>(
+      F, BNodeRules{nd}, p, [&](int k) { return S::load(src + k * p.plane + idx, p); },
+      [&](int k) { return S::load(src + k * p.plane + idx - CX[k] - CY[k] * p.pitch, p); });
 }
 
 // Everything after the boundary rules for one node: macros (with the
@@ -1180,9 +1203,10 @@ __device__ inline void three_steps_tile(const typename S::T* __restrict__ src,
 // t+1 and t+2 value they pull is formed here.  The other nodes take three
 // single steps through two more buffers; workgroups [0, nband) run the first
 // of them (k_step's work over the band and its two rings into bdst), as in
-// k_two_steps.  Not for packed lattices of instances.
+// k_two_steps.  Not for packed lattices of instances.  FP32 needs 168 VGPRs,
+// the most that leave three workgroups per CU; one more leaves two.
 template <class S, int COLL>
-__global__ __launch_bounds__(TWO_COLS) void k_three_steps(
+__global__ __launch_bounds__(TWO_COLS, S::DEV ? 3 : 1) void k_three_steps(
     const typename S::T* __restrict__ src, typename S::T* __restrict__ dst,
     const uint8_t* __restrict__ cls, const int4* __restrict__ tiles, KParams p, int nband,
     int bgrid, typename S::T* __restrict__ bdst, const uint8_t* __restrict__ bcls,

@@ -89,6 +89,31 @@ enum BNFlags : int {
   BN_DRAG = 8,        // boundary_id == drag_lift (placeholder drag/lift)
 };
 
+// Rule word of a padded cell for the LDS-resident steps: bits 0-8
+// StreamLattice, bits 9-10 the class (0: no node), above them the boundary
+// list index (LR_LIST) or, at bits 16-24, the wall links (LR_WALL).
+enum LdsRule : uint32_t {
+  LR_INTERIOR = 1u << 9,
+  LR_LIST = 2u << 9,
+  LR_WALL = 3u << 9,
+  LR_CLASS = 3u << 9,
+  LR_SHIFT = 11
+};
+// Rules of a boundary-list node for the LDS-resident steps.
+struct LdsList {
+  uint32_t bits;  // 0-8 walls (BC_ID[k] == 1), LL_*
+  uint32_t node;  // its record (cut distances)
+  double uo;
+};
+enum LdsListBits : uint32_t { LL_LID = 1u << 9, LL_WEST = 1u << 10, LL_EAST = 1u << 11 };
+// One block of the LDS-resident steps, in padded coordinates.
+struct LdsTile {
+  int x0, y0, x1, y1;      // output nodes [x0, x1) x [y0, y1); empty: padding
+  int rx0, ry0, rx1, ry1;  // cells outside hold no node of the block's lattice
+  int inst;                // batched instance (-1: the solver's parameters)
+  int plain;               // every cell of the region is an interior node
+};
+
 // Outputs of an observe pass / residual pass.
 struct KOut {
   double* rho;      // padded [plane] macro outputs (observe)

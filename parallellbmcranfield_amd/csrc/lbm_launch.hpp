@@ -29,6 +29,10 @@ struct Launch {
   const uint8_t* bcls = nullptr;
   const uint8_t* btflag = nullptr;
   const uint32_t* blist = nullptr;
+  const uint32_t* rule = nullptr;  // LDS-resident steps: rule word of each padded cell
+  const LdsTile* lds_tiles = nullptr;
+  const LdsList* lds_list = nullptr;
+  int nlds = 0, lds_shape = 0, lds_halo = 0, lds_steps = 0;
   KParams kp{};
   KOut out{};
   hipStream_t stream = nullptr;
@@ -43,9 +47,16 @@ enum Pass {
   PASS_OUTLET = 2,
   PASS_FUSED = 3,
   PASS_TWO = 4,
-  PASS_THREE = 5
+  PASS_THREE = 5,
+  PASS_LDS = 6
 };
 enum Mode { MODE_STEP = 0, MODE_RESID = 1, MODE_OBSERVE = 2 };
+
+// Region shapes of the LDS-resident steps (RX x RY nodes per workgroup).
+struct LdsShape {
+  int rx, ry;
+};
+constexpr LdsShape LDS_SHAPES[] = {{32, 16}, {32, 32}, {64, 32}};
 
 // prec: 0 F64, 1 F32, 2 F16.  coll: 1 BGKW, 2 TRT, 3 MRT.
 hipError_t launch_pass(int prec, int coll, int mode, int pass, const Launch& L);

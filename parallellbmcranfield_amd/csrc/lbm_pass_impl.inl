@@ -2,6 +2,7 @@
 #pragma once
 #include <type_traits>
 #include "lbm_kernels.inl"
+#include "lbm_lds_steps.inl"
 #include "lbm_launch.hpp"
 
 namespace lbmdev {
@@ -46,6 +47,27 @@ static hipError_t fused_launch(const Launch& L) {
   return hipGetLastError();
 }
 
+template <class S, int COLL>
+static hipError_t lds_launch(const Launch& L) {
+  using T = typename S::T;
+  const T* src = (const T*)L.src;
+  T* dst = (T*)L.dst;
+  if (L.nlds <= 0) return hipSuccess;
+  const auto go = [&](auto kernel, int nt) {
+    kernel<<<L.nlds, nt, 0, L.stream>>>(src, dst, L.rule, L.lds_tiles, L.lds_list, L.bn, L.lds_halo,
+                                        L.lds_steps, L.kp);
+    return hipGetLastError();
+  };
+  switch (L.lds_shape) {
+    case 0: return go(k_lds_steps<S, COLL, 512, 32, 1, 1>, 512);
+    case 1: return go(k_lds_steps<S, COLL, 512, 32, 2, 4>, 512);
+    case 2:
+      if constexpr (S::DEV) return go(k_lds_steps<S, COLL, 1024, 64, 2, 8>, 1024);
+      break;
+  }
+  return hipErrorInvalidValue;
+}
+
 template <class S, int COLL, int MODE>
 static hipError_t pass_mode(int pass, const Launch& L) {
   using T = typename S::T;
@@ -80,6 +102,9 @@ static hipError_t pass_mode(int pass, const Launch& L) {
             L.nbn, L.blist, L.out);
         return hipGetLastError();
       }
+      return hipErrorInvalidValue;
+    case PASS_LDS:
+      if constexpr (MODE == 0) return lds_launch<S, COLL>(L);
       return hipErrorInvalidValue;
     case PASS_OUTLET:
       if (L.norows <= 0) return hipSuccess;

@@ -302,6 +302,162 @@ static int rebuild_two_tiles(lbm_solver* s) {
   return LBM_OK;
 }
 
+// ---- several plain steps per launch, blocks of nodes in LDS
+// The blocks of running instances (all blocks of a single lattice) in launch
+// order: dealt to the XCDs in contiguous row-major runs as rebuild_two_tiles
+// deals its tiles, so that blocks that share halo lines, and the cache lines
+// that two blocks store parts of, meet in one L2.  (Runs of 4 x 4, 8 x 8 and
+// 16 x 16 blocks measured slower: 4097^2 FP32 75.2, 73.4 and 72.6 against 70.3
+// us per step.)
+static std::vector<LdsTile> lds_launch_order(const lbm_solver* s) {
+  std::vector<LdsTile> run;
+  for (const LdsTile& t : s->lds_all)
+    if (t.inst < 0 || s->inst_active[(size_t)t.inst]) run.push_back(t);
+  const int nr = (int)run.size(), q = (nr + 7) / 8;
+  LdsTile none;
+  std::memset(&none, 0, sizeof none);
+  std::vector<LdsTile> order((size_t)8 * q, none);
+  for (int x = 0; x < 8; x++)
+    for (int k = 0; k < q; k++)
+      if (x * q + k < nr) order[(size_t)8 * k + x] = run[(size_t)x * q + k];
+  return order;
+}
+
+static int rebuild_lds_tiles(lbm_solver* s) {
+  const std::vector<LdsTile> order = lds_launch_order(s);
+  if (!order.empty())
+    HC(hipMemcpyAsync(s->d_lds_tiles, order.data(), sizeof(LdsTile) * order.size(),
+                      hipMemcpyHostToDevice, s->stream));
+  HC(hipStreamSynchronize(s->stream));
+  s->nlds = (int)order.size();
+  return LBM_OK;
+}
+
+// Region shape and halo (a launch makes at most halo + 1 steps), by the
+// lattice's size.  Small lattices are bound by the latency of a launch and of
+// its steps: small regions, as many workgroups as CUs, and as many steps per
+// launch as still leave a few rows of output.  From a few hundred thousand
+// cells the chip is full and the nodes formed more than once weigh most:
+// larger regions and fewer steps, fewest where a step moves least (FP16) or
+// a node costs most (stochastic rounding).  FP64 keeps 32 x 32 (64 x 32
+// leaves one workgroup per CU).  Measured, us per step, regions 32 x 16 /
+// 32 x 32 / 64 x 32 at their best halo: FP64 BGK 129^2 1.50 / 2.88 / 4.1,
+// 361^2 2.75 / 3.5 / -, 725^2 7.9 / 7.7 / -, 1025^2 13.2 / 12.7 / 14.7; FP32
+// MRT 129^2 1.20 / 1.96 / 2.8, 361^2 1.91 / 2.38 / 2.9, 725^2 4.98 / 4.65 /
+// 4.42, 1025^2 8.8 / 7.9 / 6.7; FP16 BGK 725^2 3.89 / 3.99 / 4.18, 1449^2 - /
+// 11.4 / 10.3.  Packed lattices, whose many walls weigh more in larger
+// regions: 48 cavities, 1.3 M nodes, FP32 14.1 / 12.5 / 13.3.
+static void pick_lds_shape(lbm_solver* s, long long cells) {
+  const bool f64 = s->prec == LBM_PREC_F64, sr = s->prec == LBM_PREC_F16_SR;
+  if (cells < 25000) {
+    s->lds_shape = 0;
+    s->lds_halo = 6;
+  } else if (cells < 100000) {
+    s->lds_shape = 0;
+    s->lds_halo = f64 || sr ? 4 : 5;
+  } else if (cells < (sr ? 1200000 : 400000)) {
+    s->lds_shape = 0;
+    s->lds_halo = sr ? 2 : 3;
+  } else if (f64 || (s->ninst && !sr)) {
+    s->lds_shape = 1;
+    s->lds_halo = 4;
+  } else {
+    s->lds_shape = 2;
+    s->lds_halo = s->prec == LBM_PREC_F32 ? (cells < 900000 ? 5 : 4) : 3;
+  }
+}
+
+// Every class of nodes but open outlets, whose rows depend on each other
+// within a step.  FP16 storage with a scale that is a power of two (its
+// blocks stay in stored units).
+static int setup_lds_steps(lbm_solver* s, const std::vector<uint8_t>& cls,
+                           const std::vector<uint32_t>& wmask, const std::vector<BNode>& bn) {
+  const int n = s->cs->n, m = s->cs->m, pitch = s->pitch;
+  int e2 = 0;
+  if (s->norows > 0 || bn.size() >= (1u << (32 - LR_SHIFT)) ||
+      (s->elem == 2 && std::frexp(s->kp.scale_f, &e2) != 0.5f))
+    return LBM_OK;
+  pick_lds_shape(s, (long long)n * m);
+  const LdsShape sh = LDS_SHAPES[s->lds_shape];
+  const int h = s->lds_halo, bw = sh.rx - 2 * h, bh = sh.ry - 2 * h;
+  std::vector<int> rects;
+  if (s->ninst)
+    for (int k = 0; k < s->ninst; k++) {
+      const int* r = &s->cs->inst_rect[4 * (size_t)k];
+      rects.insert(rects.end(), {r[0] + 1, r[1] + 1, r[0] + 1 + r[2], r[1] + 1 + r[3]});
+    }
+  else
+    rects = {0, 0, n + 2, m + 2};
+  s->lds_all.clear();
+  for (size_t k = 0; 4 * k < rects.size(); k++) {
+    const int *r = &rects[4 * k];
+    // The ring of a rectangle holds no node: a lattice's is padding; a packed
+    // instance's might (a mesh whose outermost cells are fluid).
+    for (int y = r[1]; y < r[3] && s->ninst; y++)
+      for (int x = r[0]; x < r[2]; x += (y == r[1] || y == r[3] - 1) ? 1 : r[2] - r[0] - 1)
+        if (cls[(size_t)y * pitch + x] != 0) return LBM_OK;
+    for (int y = r[1] + 1; y < r[3] - 1; y += bh)
+      for (int x = r[0] + 1; x < r[2] - 1; x += bw) {
+        LdsTile t;
+        t.x0 = x;
+        t.y0 = y;
+        t.x1 = std::min(x + bw, r[2] - 1);
+        t.y1 = std::min(y + bh, r[3] - 1);
+        t.rx0 = r[0];
+        t.ry0 = r[1];
+        t.rx1 = r[2];
+        t.ry1 = r[3];
+        t.inst = s->ninst ? (int)k : -1;
+        bool any = false;
+        for (int yy = t.y0; yy < t.y1 && !any; yy++)
+          for (int xx = t.x0; xx < t.x1 && !any; xx++) any = cls[(size_t)yy * pitch + xx] != 0;
+        if (!any) continue;
+        bool plain = x - h >= r[0] && y - h >= r[1] && t.x1 + h <= r[2] && t.y1 + h <= r[3];
+        for (int yy = y - h; yy < t.y1 + h && plain; yy++)
+          for (int xx = x - h; xx < t.x1 + h && plain; xx++)
+            plain = cls[(size_t)yy * pitch + xx] == 1;
+        t.plain = plain ? 1 : 0;
+        s->lds_all.push_back(t);
+      }
+  }
+  if (s->lds_all.empty()) return LBM_OK;
+  // rule words, list rules and blocks in one allocation and one upload (three
+  // of each cost a small lattice's set-up 80 us more)
+  const std::vector<LdsTile> order = lds_launch_order(s);
+  auto round = [](size_t b) { return (b + 255) / 256 * 256; };
+  const size_t at_list = round(sizeof(uint32_t) * (size_t)s->plane);
+  const size_t at_tiles = at_list + round(sizeof(LdsList) * bn.size());
+  std::vector<char> up(at_tiles + sizeof(LdsTile) * order.size(), 0);
+  uint32_t* rule = (uint32_t*)up.data();
+  LdsList* list = (LdsList*)(up.data() + at_list);
+  std::memcpy(up.data() + at_tiles, order.data(), sizeof(LdsTile) * order.size());
+  for (size_t i = 0; i < cls.size(); i++) {
+    if (cls[i] == 1) rule[i] = LR_INTERIOR | 0x1ffu;
+    if (cls[i] == 4) rule[i] = LR_WALL | wmask[i];
+  }
+  for (size_t b = 0; b < bn.size(); b++) {
+    const BNode& nd = bn[b];
+    rule[(size_t)nd.idx] = LR_LIST | (nd.stream & 0x1ffu) | ((uint32_t)b << LR_SHIFT);
+    LdsList& l = list[b];
+    l.bits = 0;
+    for (int k = 0; k < 9; k++)
+      if (nd.bc[k] == 1) l.bits |= 1u << k;
+    const bool inlet = nd.boundary == 2 && nd.corner != 1;
+    if (inlet && nd.bc[2] == 2) l.bits |= LL_LID;
+    if (inlet && nd.bc[3] == 2) l.bits |= LL_WEST;
+    if (nd.bc[1] == 3) l.bits |= LL_EAST;
+    l.node = (uint32_t)b;
+    l.uo = nd.uo;
+  }
+  int rc = dev_alloc(s, (void**)&s->d_rule, up.size());
+  if (!rc) rc = check_hip(hipMemcpy(s->d_rule, up.data(), up.size(), hipMemcpyHostToDevice), "upload rule words");
+  s->d_lds_list = (LdsList*)((char*)s->d_rule + at_list);
+  s->d_lds_tiles = (LdsTile*)((char*)s->d_rule + at_tiles);
+  s->nlds = (int)order.size();
+  s->lds = !rc;
+  return rc;
+}
+
 static int setup_two_step(lbm_solver* s, const std::vector<uint8_t>& cls, int BS, int align,
                           long long active, const std::vector<uint16_t>& node_inst) {
   const lbm_options* o = &s->opt;
@@ -1043,6 +1199,15 @@ static int solver_create(const lbm_case* c, const lbm_options* o, const double* 
       return rc;
     }
   }
+  if (s->fused && !s->use_graph && !(o->tune_flags & LBM_TUNE_NO_TWO_STEP) &&
+      o->two_step_rows == 0 && o->three_step_rows == 0) {
+    rc = setup_lds_steps(s, cls, wmask, bn);
+    if (rc) {
+      if (d_grad) (void)hipFree(d_grad);
+      lbm_solver_destroy(s);
+      return rc;
+    }
+  }
   if (s->prec != LBM_PREC_F16_SR && !(o->tune_flags & LBM_TUNE_NO_TWO_STEP)) {
     long long active = 0;
     for (uint8_t cv : cls) active += cv != 0;
@@ -1253,6 +1418,24 @@ static int build_graph(lbm_solver* s, int parity) {
   return check_hip(e, "hipGraphInstantiate");
 }
 
+// `steps` plain steps (2 .. halo + 1) from buf[src_buf] into buf[src_buf ^ 1].
+static int launch_lds_steps(lbm_solver* s, int src_buf, int steps, hipEvent_t e0 = nullptr,
+                            hipEvent_t e1 = nullptr) {
+  Launch L = make_launch(s, src_buf);
+  L.kp.res_kind = RK_NONE;
+  L.rule = s->d_rule;
+  L.lds_tiles = s->d_lds_tiles;
+  L.lds_list = s->d_lds_list;
+  L.nlds = s->nlds;
+  L.lds_shape = s->lds_shape;
+  L.lds_halo = s->lds_halo;
+  L.lds_steps = steps;
+  if (e0) HC(hipEventRecord(e0, s->stream));
+  HC(pass(s, MODE_STEP, PASS_LDS, L));
+  if (e1) HC(hipEventRecord(e1, s->stream));
+  return LBM_OK;
+}
+
 extern "C" {
 
 int lbm_solver_create(const lbm_case* c, const lbm_options* o, lbm_solver** out) {
@@ -1301,7 +1484,7 @@ void lbm_solver_destroy(lbm_solver* s) {
                   s->d_tflag_b[0], s->d_tflag_b[1], s->d_list_b[0], s->d_list_b[1],
                   s->d_tiles3, s->d_cls_three, s->buf4, s->d_cls_b3[0], s->d_cls_b3[1],
                   s->d_cls_b3[2], s->d_tflag_b3[0], s->d_tflag_b3[1], s->d_tflag_b3[2],
-                  s->d_list_b3[0], s->d_list_b3[1], s->d_list_b3[2]};
+                  s->d_list_b3[0], s->d_list_b3[1], s->d_list_b3[2], s->d_rule};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (hipEvent_t e : s->ev) (void)hipEventDestroy(e);
@@ -1344,6 +1527,10 @@ static int rebuild_tile_list(lbm_solver* s) {
       (void)hipGraphExecDestroy(g);
       g = nullptr;
     }
+  if (s->lds) {
+    int rc = rebuild_lds_tiles(s);
+    if (rc) return rc;
+  }
   if (s->two) return rebuild_two_tiles(s);
   return LBM_OK;
 }
@@ -1458,6 +1645,40 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
     // (256-cavity sweep 25.6 k against 51.4 k MLUPS aggregate), and a small
     // lattice's launches are faster direct than replayed two to a graph (129^2
     // under its stop rule 8.1 against 5.7 us per step).
+    // A run of plain steps with LDS-resident blocks.  The last step of a call
+    // (and the last before the iteration cap) is a single one, so that
+    // observe passes and checkpoints find the state one step back.  Runs of
+    // two on lattices with two- and three-step launches go to those (with the
+    // single step after them, us: 4097^2 FP32 403 for a three-step launch
+    // against 613, FP64 2049^2 254 against 317).
+    if (s->lds && !eval) {
+      const int most = s->lds_halo + 1;
+      const int least = (s->two || s->three) && (long long)s->cs->n * s->cs->m >= (1LL << 22) ? 3 : 2;
+      int run = 1;  // looked ahead as far as the length of this launch depends on it
+      while (run < 2 * most && t + run < nsteps && !evals_at(s->iter + run) &&
+             !forces_at(s->iter + run) &&
+             (!o.use_stop_rule || s->iter + run < o.max_iterations))
+        run++;
+      if (t + run == nsteps || (o.use_stop_rule && s->iter + run == o.max_iterations)) run--;
+      if (run >= least) {
+        // the last launches of a run share it equally
+        const int k = run >= 2 * most - 1 ? most : (run > most ? (run + 1) / 2 : run);
+        int ts = t;  // a sampled step in this launch
+        while (evs && ts < t + k && ts % sample_every) ts++;
+        const bool sample = evs && ts < t + k;
+        const size_t ei = sample ? 2 * (size_t)(ts / sample_every) : 0;
+        int rc = launch_lds_steps(s, s->cur, k, sample ? (*evs)[ei] : nullptr,
+                                  sample ? (*evs)[ei + 1] : nullptr);
+        if (rc) return rc;
+        if (sample && rec) rec->push_back(ei);
+        s->cur ^= 1;
+        s->iter += k;
+        ran += k;
+        t += k - 1;
+        s->prev_stale = false;
+        continue;
+      }
+    }
     const bool runs_ok = !stop_can_trigger || (!s->ninst && (s->two || s->three));
     const bool plain_pair = t + 1 < nsteps && !eval && !evals_at(s->iter + 1) &&
                             !forces_at(s->iter + 1) && runs_ok &&
@@ -1540,8 +1761,9 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
     L.kp.res_kind = rpart ? (rk == LBM_RESID_FULL ? RK_FULL : RK_VEL) : RK_NONE;
     L.kp.force_on = feval ? 1 : 0;
     if (rk == LBM_RESID_REFERENCE) L.out.cres = s->d_cres;
-    // with multi-step launches only those are sampled
-    const bool timed = evs && !s->two && !s->three && (t % sample_every == 0);
+    // with multi-step launches only those are sampled (runs too short for one aside)
+    const bool timed = evs && !s->two && !s->three && (!s->lds || nsteps < 3) &&
+                       (t % sample_every == 0);
     const size_t ei = 2 * (size_t)(t / (sample_every > 0 ? sample_every : 1));
     if (timed) HC(hipEventRecord((*evs)[ei], s->stream));
     if (timed && rec) rec->push_back(ei);
@@ -1756,7 +1978,7 @@ size_t lbm_solver_device_bytes(const lbm_solver* s) { return s ? s->dev_bytes : 
 int lbm_solver_fused(const lbm_solver* s) {
   if (!s) return 0;
   return (s->fused ? 1 : 0) | (make_launch(const_cast<lbm_solver*>(s), 0).pairs ? 2 : 0) |
-         (s->two ? 4 : 0) | (s->three ? 8 : 0);
+         (s->two ? 4 : 0) | (s->three ? 8 : 0) | (s->lds ? (s->lds_halo + 1) << 8 : 0);
 }
 
 int lbm_solver_two_step_info(const lbm_solver* s, long long* cells, int* tiles, int* rows,

@@ -141,7 +141,7 @@ def _time_steps(case: Case, o, instances, steps: int) -> tuple[float, dict, dict
     are captured on first use), and the solver's multi-step layout."""
     s = Solver(case, o, instances=instances) if instances else Solver(case, o)
     try:
-        two, three = s.two_step_info(), s.three_step_info()
+        two, three = dict(s.two_step_info(), lds_steps=s.lds_steps), s.three_step_info()
         s.step(24)
         s.sync()
         t0 = time.perf_counter()
@@ -169,8 +169,8 @@ def autotune(case: Case, opts, instances=None, steps: int = 198,
     Stage 2: at the best stage-1 shape, the tile shape of multi-step
     launches: two plain steps per launch with `two_rows` output rows per
     256-column tile, three per launch with `three_rows` (single lattices
-    only; 0: the library's own pick, which may be single steps where
-    multi-step launches lose), each against single steps.  A variant whose
+    only; 0: the library's own pick, runs of steps with LDS-resident blocks
+    where it has them), each against single steps.  A variant whose
     solver runs no such launches is dropped.  `best` holds the options to
     copy (block_size, xcd_group, two_step_rows, three_step_rows, tune_flags)
     and what ran."""
@@ -189,7 +189,8 @@ def autotune(case: Case, opts, instances=None, steps: int = 198,
         return o
 
     def record(o, dt, two, three, stage):
-        steps_per_launch = 3 if three["cells"] else (2 if two["cells"] else 1)
+        steps_per_launch = two.get("lds_steps") or (3 if three["cells"] else
+                                                    (2 if two["cells"] else 1))
         return dict(stage=stage, block_size=o.block_size, xcd_group=o.xcd_group,
                     pairs=fp16 and o.block_size == 256 and not (o.tune_flags & TUNE_NO_PAIRS),
                     two_step_rows=o.two_step_rows, three_step_rows=o.three_step_rows,
@@ -210,7 +211,7 @@ def autotune(case: Case, opts, instances=None, steps: int = 198,
     for r2 in two_rows:
         o = variant(best1["block_size"], best1["xcd_group"], base | TUNE_NO_THREE_STEP, rows2=r2)
         dt, two, three = _time_steps(case, o, instances, steps)
-        if two["cells"]:
+        if two["cells"] or two.get("lds_steps"):
             results.append(record(o, dt, two, three, 2))
     for r3 in (() if instances else three_rows):
         o = variant(best1["block_size"], best1["xcd_group"], base, rows3=r3)
