@@ -82,6 +82,9 @@ struct lbm_solver {
   double* d_metaf = nullptr;  // padded [9][plane] (allocated on demand)
   double* d_snap = nullptr;   // velocity residual snapshot [3][plane]
   double* d_cres = nullptr;   // [m][12]
+  // the reference residual's cells (the first m) hold no node, so that every
+  // row of it is zero, and no stop rule reads it: no step evaluates it
+  bool ref_zero = false;
   double* d_part = nullptr;   // [nparts][4]
   double* d_hist = nullptr;   // [HCAP][4]
   uint32_t* d_seed = nullptr; // FP16 stochastic rounding: step number, 2 slots

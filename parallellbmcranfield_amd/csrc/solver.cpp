@@ -932,6 +932,10 @@ static int solver_create(const lbm_case* c, const lbm_options* o, const double* 
   orow.push_back((int)on.size());
   s->nbn = (int)bn.size();
   s->non = (int)on.size();
+  s->ref_zero = s->opt.resid_kind == LBM_RESID_REFERENCE &&
+                !(o->use_stop_rule && (o->crit_v >= 0 || o->crit_rho >= 0));
+  for (const std::vector<BNode>* v : {&bn, &on})
+    for (const BNode& b : *v) s->ref_zero = s->ref_zero && !(b.flags & BN_COMPAT_RES);
   s->norows = (int)orow.size() - 1;
   s->nside = nside;
 
@@ -1052,7 +1056,7 @@ static int solver_create(const lbm_case* c, const lbm_options* o, const double* 
     if (!rc) rc = check_hip(hipMemset(s->d_seed, 0, 2 * sizeof(uint32_t)), "clear step number");
     kp.seed = s->d_seed;
   }
-  if (!rc && s->opt.resid_kind == LBM_RESID_REFERENCE)
+  if (!rc && s->opt.resid_kind == LBM_RESID_REFERENCE && !s->ref_zero)
     rc = dev_alloc(s, (void**)&s->d_cres, sizeof(double) * 12 * (size_t)m);
   if (!rc && s->opt.resid_kind == LBM_RESID_VELOCITY)
     rc = dev_alloc(s, (void**)&s->d_snap, sizeof(double) * (ninst ? 5 : 3) * (size_t)s->plane);
@@ -1614,6 +1618,16 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
   const bool stop_can_trigger = o.use_stop_rule && (o.crit_v >= 0 || o.crit_rho >= 0);
   const int K = o.resid_every;
   int ran = 0;
+  // k steps done; a reference residual that is always zero gives their rows
+  auto made = [&](int k) {
+    if (s->ref_zero) {
+      for (int i = 0; i < k; i++) s->hist_iter.push_back(s->iter + i);
+      s->hist_val.insert(s->hist_val.end(), 4 * (size_t)k, 0.0);
+      std::memset(s->resid, 0, sizeof s->resid);
+    }
+    s->iter += k;
+    ran += k;
+  };
   for (int t = 0; t < nsteps; t++) {
     if (o.use_stop_rule) {
       if (stop_can_trigger) {
@@ -1626,7 +1640,7 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
     }
     const int rk = o.resid_kind;
     auto evals_at = [&](int it) {  // does the step that ends at iteration it+1 evaluate?
-      return rk == LBM_RESID_REFERENCE ||
+      return (rk == LBM_RESID_REFERENCE && !s->ref_zero) ||
              ((rk == LBM_RESID_FULL || rk == LBM_RESID_VELOCITY) && (it + 1) % K == 0);
     };
     const bool reval = evals_at(s->iter);
@@ -1672,8 +1686,7 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
         if (rc) return rc;
         if (sample && rec) rec->push_back(ei);
         s->cur ^= 1;
-        s->iter += k;
-        ran += k;
+        made(k);
         t += k - 1;
         s->prev_stale = false;
         continue;
@@ -1709,8 +1722,7 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
         if (rc) return rc;
       }
       s->cur ^= 1;
-      s->iter += 3;
-      ran += 3;
+      made(3);
       t += 2;
       s->prev_stale = true;
       s->prev_lag = 3;
@@ -1735,8 +1747,7 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
         if (rc) return rc;
       }
       s->cur ^= 1;
-      s->iter += 2;
-      ran += 2;
+      made(2);
       t += 1;
       s->prev_stale = true;
       s->prev_lag = 2;
@@ -1750,8 +1761,7 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
         if (rc) return rc;
       }
       HC(hipGraphLaunch(s->gexec[s->cur], s->stream));
-      s->iter += 2;
-      ran += 2;
+      made(2);
       t += 1;
       continue;
     }
@@ -1787,8 +1797,7 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
       s->pending++;
     }
     s->cur ^= 1;
-    s->iter++;
-    ran++;
+    made(1);
     if (s->ninst && reval) {
       int rc = batch_eval(s);
       if (rc) {
