@@ -72,6 +72,9 @@ struct lbm_solver {
   uint32_t* d_wmask = nullptr;  // class-4 (in-tile wall) cells: stream and wall-link bits
   lbmdev::BNode* d_bn = nullptr;
   int nbn = 0;
+  int* d_body = nullptr;        // runs of 256 boundary-list nodes that hold the force body's
+  int nbody = 0;
+  bool force_pass = false;      // force steps are plain steps after a k_force launch
   lbmdev::BNode* d_on = nullptr;
   int* d_orow = nullptr;
   int norows = 0, non = 0;

@@ -33,6 +33,9 @@ struct Launch {
   const LdsTile* lds_tiles = nullptr;
   const LdsList* lds_list = nullptr;
   int nlds = 0, lds_shape = 0, lds_halo = 0, lds_steps = 0;
+  const int* body = nullptr;   // runs of 256 boundary-list nodes that hold the force body's
+  int nbody = 0;
+  double* hist = nullptr;      // history slot of a force pass
   KParams kp{};
   KOut out{};
   hipStream_t stream = nullptr;
@@ -40,7 +43,8 @@ struct Launch {
 
 // PASS_TWO / PASS_THREE: two / three plain steps of the multi-step tiles
 // (MODE_STEP, not with stochastic rounding; three: not for packed lattices
-// of instances).
+// of instances).  PASS_LDS: lds_steps plain steps (MODE_STEP).  PASS_FORCE:
+// the force of the step that reads src -> hist[4..5] (MODE_RESID).
 enum Pass {
   PASS_BULK = 0,
   PASS_BOUNDARY = 1,
@@ -48,7 +52,8 @@ enum Pass {
   PASS_FUSED = 3,
   PASS_TWO = 4,
   PASS_THREE = 5,
-  PASS_LDS = 6
+  PASS_LDS = 6,
+  PASS_FORCE = 7
 };
 enum Mode { MODE_STEP = 0, MODE_RESID = 1, MODE_OBSERVE = 2 };
 

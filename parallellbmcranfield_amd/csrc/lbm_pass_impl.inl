@@ -106,6 +106,12 @@ static hipError_t pass_mode(int pass, const Launch& L) {
     case PASS_LDS:
       if constexpr (MODE == 0) return lds_launch<S, COLL>(L);
       return hipErrorInvalidValue;
+    case PASS_FORCE:
+      if constexpr (MODE == 1 && COLL == 1) {  // the same for every collision
+        k_force<S><<<1, 1024, 0, L.stream>>>(src, L.bn, L.nbn, L.body, L.nbody, L.kp, L.hist);
+        return hipGetLastError();
+      }
+      return hipErrorInvalidValue;
     case PASS_OUTLET:
       if (L.norows <= 0) return hipSuccess;
       k_outlet<S, COLL, MODE><<<(L.norows + 63) / 64, 64, 0, L.stream>>>(

@@ -1160,6 +1160,21 @@ static int solver_create(const lbm_case* c, const lbm_options* o, const double* 
     kp.wmask = s->d_wmask;
   }
   if (!rc && s->nbn) rc = check_hip(hipMemcpy(s->d_bn, bn.data(), sizeof(BNode) * bn.size(), hipMemcpyHostToDevice), "upload boundary list");
+  // the force body (open-outlet nodes take their force in the outlet pass).
+  // A body spread over more runs than one workgroup takes in four rounds
+  // keeps the residual form.
+  if (!rc && o->force_id != 0 && o->force_every > 0 && s->norows == 0 && s->fused) {
+    std::vector<int> body;
+    for (size_t i = 0; i < bn.size(); i++)
+      if (bn[i].boundary_id == o->force_id && (body.empty() || body.back() != (int)(i / 256)))
+        body.push_back((int)(i / 256));
+    if (!body.empty() && body.size() <= 16) {
+      s->nbody = (int)body.size();
+      s->force_pass = true;
+      rc = dev_alloc(s, (void**)&s->d_body, sizeof(int) * body.size());
+      if (!rc) rc = check_hip(hipMemcpy(s->d_body, body.data(), sizeof(int) * body.size(), hipMemcpyHostToDevice), "upload force body");
+    }
+  }
   if (!rc && s->non) rc = check_hip(hipMemcpy(s->d_on, on.data(), sizeof(BNode) * on.size(), hipMemcpyHostToDevice), "upload outlet list");
   if (!rc) rc = check_hip(hipMemcpy(s->d_orow, orow.data(), sizeof(int) * orow.size(), hipMemcpyHostToDevice), "upload outlet rows");
   if (!rc && s->d_cres) rc = check_hip(hipMemset(s->d_cres, 0, sizeof(double) * 12 * (size_t)m), "clear cres");
@@ -1488,7 +1503,7 @@ void lbm_solver_destroy(lbm_solver* s) {
                   s->d_tflag_b[0], s->d_tflag_b[1], s->d_list_b[0], s->d_list_b[1],
                   s->d_tiles3, s->d_cls_three, s->buf4, s->d_cls_b3[0], s->d_cls_b3[1],
                   s->d_cls_b3[2], s->d_tflag_b3[0], s->d_tflag_b3[1], s->d_tflag_b3[2],
-                  s->d_list_b3[0], s->d_list_b3[1], s->d_list_b3[2], s->d_rule};
+                  s->d_list_b3[0], s->d_list_b3[1], s->d_list_b3[2], s->d_rule, s->d_body};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (hipEvent_t e : s->ev) (void)hipEventDestroy(e);
@@ -1647,7 +1662,24 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
     auto forces_at = [&](int it) {
       return o.force_id != 0 && o.force_every > 0 && (it + 1) % o.force_every == 0;
     };
-    const bool feval = forces_at(s->iter);
+    if (s->force_pass && forces_at(s->iter)) {
+      Launch L = make_launch(s, s->cur);
+      L.body = s->d_body;
+      L.nbody = s->nbody;
+      L.hist = s->d_hist + (size_t)s->pending * HW;
+      HC(s->prec == 0 ? launch_pass_f64(1, MODE_RESID, PASS_FORCE, L)
+                      : launch_pass_lp(s->prec, 1, MODE_RESID, PASS_FORCE, L));
+      s->pending_iter.push_back(s->iter);
+      s->pending_what.push_back(2);
+      if (++s->pending == HCAP) {
+        int rc = flush_history(s);
+        if (rc) {
+          if (done) *done = ran;
+          return rc;
+        }
+      }
+    }
+    const bool feval = !s->force_pass && forces_at(s->iter);
     const bool eval = reval || feval;
     // The stop rule reads only evaluated residuals, which change at
     // evaluation steps alone, and a run of plain steps holds none: the rule
