@@ -44,6 +44,7 @@ UNITS = [
     ("residuals.hip", "hip", ["-ffp-contract=off"]),
     ("residuals_noalloc.hip", "hip", ["-ffp-contract=off"]),
     ("nn_kernels.hip", "hip", ["-mllvm", "-amdgpu-mfma-vgpr-form"]),
+    ("transfer.hip", "hip", []),
     ("case_io.cpp", "host", []),
     ("solver.cpp", "host", []),
     ("run.cpp", "host", []),

@@ -8,6 +8,7 @@
 
 #include "../../include/lbm.h"
 #include "lbm_kparams.hpp"
+#include "transfer.hpp"
 
 namespace lbmhost {
 
@@ -60,6 +61,7 @@ struct lbm_solver {
   lbm_options opt{};
   int prec = 0, coll = 1;
   hipStream_t stream = nullptr;
+  lbmhost::Staging staging;  // pinned slots of the copies to the caller's arrays
   int device = 0;
   // layout
   int pitch = 0, rows = 0, plane = 0;

@@ -17,10 +17,13 @@
 // head W[3][c] then b[3].  The first conv's Cin is padded from 3 to 32.
 //
 // No counterpart in the reference.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/lbm.h"
@@ -53,6 +56,9 @@ struct lbm_net {
   float div_w = 0.0f, div_su = 1.0f, div_sv = 1.0f;  // divergence penalty of the loss
   int dil = 1;  // bottleneck dilation: its convs use dil and 2 dil
   hipStream_t st = nullptr;
+  hipStream_t cs = nullptr;  // copies that run beside the kernels of st
+  hipEvent_t ev_st = nullptr, ev_cs = nullptr;  // a point of st (of cs) that the other waits for
+  lbmhost::Staging staging;
   std::vector<Conv> conv;
   size_t nparam = 0, head_w = 0, head_b = 0;
   float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;  // FP32 master, grad, Adam
@@ -68,7 +74,8 @@ struct lbm_net {
   float* part = nullptr;
   size_t part_cap = 0;
   int* idx = nullptr;
-  float *stage_in = nullptr, *stage_t = nullptr;  // host-batch staging [Bmax][H][W][3]
+  float* stage_in = nullptr;  // a host batch [Bmax][H][W][cin]
+  float* stage_y = nullptr;   // a batch's predictions on their way to the host [Bmax][H][W][3]
   // training set
   float *set_in = nullptr, *set_t = nullptr;
   int nset = 0;
@@ -179,6 +186,9 @@ int lbm_net_create(int H, int W, int batch, int base, int levels, int in_channel
   n->nparam = off;
 
   int rc = check_hip(hipStreamCreateWithFlags(&n->st, hipStreamNonBlocking), "hipStreamCreate");
+  if (!rc) rc = check_hip(hipStreamCreateWithFlags(&n->cs, hipStreamNonBlocking), "hipStreamCreate");
+  if (!rc) rc = check_hip(hipEventCreateWithFlags(&n->ev_st, hipEventDisableTiming), "hipEventCreate");
+  if (!rc) rc = check_hip(hipEventCreateWithFlags(&n->ev_cs, hipEventDisableTiming), "hipEventCreate");
   if (!rc) rc = nalloc_t(n, &n->p, off);
   if (!rc) rc = nalloc_t(n, &n->g, off);
   if (!rc) rc = nalloc_t(n, &n->m, off);
@@ -225,7 +235,7 @@ int lbm_net_create(int H, int W, int batch, int base, int levels, int in_channel
   if (!rc) rc = nalloc_t(n, &n->dvpart, (P0 + 255) / 256);
   if (!rc) rc = nalloc_t(n, &n->idx, (size_t)B);
   if (!rc) rc = nalloc_t(n, &n->stage_in, P0 * in_channels);
-  if (!rc) rc = nalloc_t(n, &n->stage_t, P0 * 3);
+  if (!rc) rc = nalloc_t(n, &n->stage_y, P0 * 3);
   // partial-sum scratch: the largest conv weight-gradient partials, the
   // bias and head partials
   size_t cap = 0;
@@ -275,13 +285,52 @@ int lbm_net_create(int H, int W, int batch, int base, int levels, int in_channel
 
 void lbm_net_destroy(lbm_net* n) {
   if (!n) return;
-  if (n->st) (void)hipStreamSynchronize(n->st);
+  for (hipStream_t st : {n->st, n->cs})
+    if (st) (void)hipStreamSynchronize(st);
   for (void* q : n->allocs) (void)hipFree(q);
-  if (n->st) (void)hipStreamDestroy(n->st);
+  for (hipEvent_t ev : {n->ev_st, n->ev_cs})
+    if (ev) (void)hipEventDestroy(ev);
+  for (hipStream_t st : {n->st, n->cs})
+    if (st) (void)hipStreamDestroy(st);
   delete n;
 }
 
 long lbm_net_num_params(const lbm_net* n) { return n ? (long)n->nparam : -1; }
+
+// `unit` floats of each of `count` items between a caller's array and the device
+static int to_device(lbm_net* n, hipStream_t st, const float* src, float* dst, size_t count,
+                     size_t unit) {
+  NC(n->staging.to_device(
+      st, count, sizeof(float) * unit,
+      [&](size_t off, size_t len, char* slot) {
+        std::memcpy(slot, src + off * unit, sizeof(float) * len * unit);
+      },
+      [&](size_t off, size_t len, char* slot) {
+        const void* from = slot;
+        return n->staging.copy(dst + off * unit, &from, 1, sizeof(float) * len * unit, st);
+      }));
+  return LBM_OK;
+}
+
+static int to_host(lbm_net* n, hipStream_t st, const float* src, float* dst, size_t count) {
+  NC(n->staging.to_host(
+      st, count, sizeof(float),
+      [&](size_t off, size_t len, char* slot) {
+        const void* from = src + off;
+        return n->staging.copy(slot, &from, 1, sizeof(float) * len, st);
+      },
+      [&](size_t off, size_t len, char* slot) {
+        std::memcpy(dst + off, slot, sizeof(float) * len);
+      }));
+  return LBM_OK;
+}
+
+// Work queued on `later` from here on starts after what `first` holds now.
+static int order(hipStream_t first, hipStream_t later, hipEvent_t ev) {
+  NC(hipEventRecord(ev, first));
+  NC(hipStreamWaitEvent(later, ev, 0));
+  return LBM_OK;
+}
 
 static int refresh_weights(lbm_net* n) {
   NC(to_bf16(n->p, n->pb, (long)n->nparam, n->st));
@@ -291,11 +340,12 @@ static int refresh_weights(lbm_net* n) {
 
 int lbm_net_set_params(lbm_net* n, const float* params) {
   if (!n || !params) return LBM_EINVAL;
-  NC(hipMemcpyAsync(n->p, params, sizeof(float) * n->nparam, hipMemcpyHostToDevice, n->st));
+  int rc = to_device(n, n->st, params, n->p, n->nparam, 1);
+  if (rc) return rc;
   NC(hipMemsetAsync(n->m, 0, sizeof(float) * n->nparam, n->st));
   NC(hipMemsetAsync(n->v, 0, sizeof(float) * n->nparam, n->st));
   n->step = 0;
-  int rc = refresh_weights(n);
+  rc = refresh_weights(n);
   if (rc) return rc;
   NC(hipStreamSynchronize(n->st));
   return LBM_OK;
@@ -303,9 +353,7 @@ int lbm_net_set_params(lbm_net* n, const float* params) {
 
 int lbm_net_get_params(lbm_net* n, float* params) {
   if (!n || !params) return LBM_EINVAL;
-  NC(hipMemcpyAsync(params, n->p, sizeof(float) * n->nparam, hipMemcpyDeviceToHost, n->st));
-  NC(hipStreamSynchronize(n->st));
-  return LBM_OK;
+  return to_host(n, n->st, n->p, params, n->nparam);
 }
 
 // forward of B samples already in x0
@@ -427,12 +475,9 @@ static int backward(lbm_net* n, int B, double fluid, double* loss) {
   }
   if (loss) {
     std::vector<float> lp((size_t)(P0 + 255) / 256), dp(lp.size(), 0.0f);
-    NC(hipMemcpyAsync(lp.data(), n->lpart, sizeof(float) * lp.size(), hipMemcpyDeviceToHost,
-                      n->st));
-    if (n->div_w > 0.0f)
-      NC(hipMemcpyAsync(dp.data(), n->dvpart, sizeof(float) * dp.size(), hipMemcpyDeviceToHost,
-                        n->st));
-    NC(hipStreamSynchronize(n->st));
+    int rc = to_host(n, n->st, n->lpart, lp.data(), lp.size());
+    if (!rc && n->div_w > 0.0f) rc = to_host(n, n->st, n->dvpart, dp.data(), dp.size());
+    if (rc) return rc;
     double sum = 0.0, dsum = 0.0;
     for (float f : lp) sum += f;
     for (float f : dp) dsum += f;
@@ -441,56 +486,82 @@ static int backward(lbm_net* n, int B, double fluid, double* loss) {
   return LBM_OK;
 }
 
-// x0 / t / mask from host arrays (nb <= Bmax samples, [H][W][3] each)
-static int upload_batch(lbm_net* n, const float* in, const float* tg, int nb, double* fluid) {
-  const size_t HW = (size_t)n->H * n->W;
-  std::vector<int> id(nb);
-  for (int b = 0; b < nb; b++) id[b] = b;
-  NC(hipMemcpyAsync(n->stage_in, in, sizeof(float) * HW * n->cin * nb, hipMemcpyHostToDevice,
-                    n->st));
-  if (tg)
-    NC(hipMemcpyAsync(n->stage_t, tg, sizeof(float) * HW * 3 * nb, hipMemcpyHostToDevice, n->st));
-  NC(hipMemcpyAsync(n->idx, id.data(), sizeof(int) * nb, hipMemcpyHostToDevice, n->st));
-  NC(gather(n->stage_in, n->stage_t, n->idx, n->x0, tg ? n->t : nullptr, tg ? n->mask : nullptr,
-            nb, (int)HW, n->cin, CIN0, n->st));
-  NC(hipStreamSynchronize(n->st));  // the host arrays may go after return
-  if (fluid) {
-    double f = 0.0;
-    for (size_t q = 0; q < HW * nb; q++) f += in[q * n->cin];
-    *fluid = f;
-  }
+// `count` pixels of a host batch to stage_in, and the sum of their channel 0,
+// taken while the threads read them: the blocks' sums are added in their order.
+static int upload_inputs(lbm_net* n, hipStream_t st, const float* in, size_t count,
+                         double* fluid) {
+  const size_t ci = (size_t)n->cin;
+  if (!fluid) return to_device(n, st, in, n->stage_in, count, ci);
+  std::mutex mu;
+  std::vector<std::pair<size_t, double>> part;
+  NC(n->staging.to_device(
+      st, count, sizeof(float) * ci,
+      [&](size_t off, size_t len, char* slot) {
+        std::memcpy(slot, in + off * ci, sizeof(float) * len * ci);
+        const float* p = (const float*)slot;
+        double f = 0.0;
+        for (size_t q = 0; q < len; q++) f += p[q * ci];
+        std::lock_guard<std::mutex> lock(mu);
+        part.emplace_back(off, f);
+      },
+      [&](size_t off, size_t len, char* slot) {
+        const void* from = slot;
+        return n->staging.copy(n->stage_in + off * ci, &from, 1, sizeof(float) * len * ci, st);
+      }));
+  std::sort(part.begin(), part.end());
+  *fluid = 0.0;
+  for (const auto& p : part) *fluid += p.second;
   return LBM_OK;
 }
 
+// Batches of Bmax: while the kernels of one run on st, the host takes the
+// batch before it from stage_y and sends the batch after it to stage_in, both
+// on cs.
 int lbm_net_predict(lbm_net* n, const float* in, int nb, float* out) {
   if (!n || !in || !out || nb < 0) return LBM_EINVAL;
   const size_t HW = (size_t)n->H * n->W;
-  for (int b0 = 0; b0 < nb; b0 += n->Bmax) {
-    const int B = std::min(n->Bmax, nb - b0);
-    int rc = upload_batch(n, in + HW * n->cin * b0, nullptr, B, nullptr);
-    if (rc) return rc;
-    rc = forward(n, B);
-    if (rc) return rc;
-    NC(hipMemcpyAsync(out + HW * 3 * b0, n->y, sizeof(float) * HW * 3 * B, hipMemcpyDeviceToHost,
+  const int step = n->Bmax;
+  int rc = LBM_OK;
+  if (nb > 0) rc = upload_inputs(n, n->st, in, HW * std::min(step, nb), nullptr);
+  for (int b0 = 0; b0 < nb && !rc; b0 += step) {
+    const int B = std::min(step, nb - b0);
+    NC(gather(n->stage_in, nullptr, nullptr, n->x0, nullptr, nullptr, B, (int)HW, n->cin, CIN0,
+              n->st));
+    rc = order(n->st, n->cs, n->ev_st);  // stage_in is read, and stage_y written before
+    if (!rc) rc = forward(n, B);
+    if (!rc && b0)
+      rc = to_host(n, n->cs, n->stage_y, out + HW * 3 * (size_t)(b0 - step), HW * 3 * step);
+    if (rc) break;
+    NC(hipMemcpyAsync(n->stage_y, n->y, sizeof(float) * HW * 3 * B, hipMemcpyDeviceToDevice,
                       n->st));
-    NC(hipStreamSynchronize(n->st));
+    const int next = std::min(step, nb - b0 - B);
+    if (next > 0) {
+      rc = upload_inputs(n, n->cs, in + HW * n->cin * (size_t)(b0 + B), HW * next, nullptr);
+      if (!rc) rc = order(n->cs, n->st, n->ev_cs);
+    } else {
+      rc = to_host(n, n->st, n->stage_y, out + HW * 3 * (size_t)b0, HW * 3 * B);
+    }
   }
-  return LBM_OK;
+  return rc;
 }
 
 int lbm_net_gradients(lbm_net* n, const float* in, const float* target, int nb, double* loss,
                       float* grads) {
   if (!n || !in || !target || nb < 1 || nb > n->Bmax) return LBM_EINVAL;
+  const size_t HW = (size_t)n->H * n->W;
   double fluid = 0.0;
-  int rc = upload_batch(n, in, target, nb, &fluid);
-  if (!rc) rc = forward(n, nb);
-  if (!rc) rc = backward(n, nb, fluid, loss);
+  int rc = upload_inputs(n, n->st, in, HW * nb, &fluid);
   if (rc) return rc;
-  if (grads) {
-    NC(hipMemcpyAsync(grads, n->g, sizeof(float) * n->nparam, hipMemcpyDeviceToHost, n->st));
-    NC(hipStreamSynchronize(n->st));
-  }
-  return LBM_OK;
+  NC(gather(n->stage_in, nullptr, nullptr, n->x0, nullptr, n->mask, nb, (int)HW, n->cin, CIN0,
+            n->st));
+  // the targets follow on cs, behind every reader of t so far and beside the forward
+  rc = order(n->st, n->cs, n->ev_st);
+  if (!rc) rc = forward(n, nb);
+  if (!rc) rc = to_device(n, n->cs, target, n->t, HW * nb, 3);
+  if (!rc) rc = order(n->cs, n->st, n->ev_cs);
+  if (!rc) rc = backward(n, nb, fluid, loss);
+  if (!rc && grads) rc = to_host(n, n->st, n->g, grads, n->nparam);
+  return rc;
 }
 
 int lbm_net_set_data(lbm_net* n, const float* in, const float* target, int count) {
@@ -507,8 +578,10 @@ int lbm_net_set_data(lbm_net* n, const float* in, const float* target, int count
   NC(hipMalloc((void**)&n->set_t, sizeof(float) * HW * 3 * count));
   n->allocs.push_back(n->set_in);
   n->allocs.push_back(n->set_t);
-  NC(hipMemcpy(n->set_in, in, sizeof(float) * HW * n->cin * count, hipMemcpyHostToDevice));
-  NC(hipMemcpy(n->set_t, target, sizeof(float) * HW * 3 * count, hipMemcpyHostToDevice));
+  int rc = to_device(n, n->st, in, n->set_in, HW * count, n->cin);
+  if (!rc) rc = to_device(n, n->st, target, n->set_t, HW * count, 3);
+  if (rc) return rc;
+  NC(hipStreamSynchronize(n->st));
   n->nset = count;
   n->set_fluid.assign(count, 0.0);
   for (int k = 0; k < count; k++) {

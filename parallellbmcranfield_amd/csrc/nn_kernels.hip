@@ -882,7 +882,8 @@ __global__ void k_gather(const float* __restrict__ inputs, const float* __restri
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= B * HW) return;
   const int b = i / HW, q = i % HW;
-  const size_t src = ((size_t)idx[b] * HW + q) * Ci;
+  const size_t sample = idx ? (size_t)idx[b] : (size_t)b;
+  const size_t src = (sample * HW + q) * Ci;
   float f[8];
   for (int c0 = 0; c0 < Cp; c0 += 8) {
 #pragma unroll
@@ -890,10 +891,10 @@ __global__ void k_gather(const float* __restrict__ inputs, const float* __restri
     st8(x + (size_t)i * Cp + c0, pack8(f));
   }
   if (t) {
-    const size_t ts = ((size_t)idx[b] * HW + q) * 3;
+    const size_t ts = (sample * HW + q) * 3;
     for (int c = 0; c < 3; c++) t[(size_t)i * 3 + c] = targets[ts + c];
-    mask[i] = inputs[src];
   }
+  if (mask) mask[i] = inputs[src];
 }
 
 // ------------------------------------------------------------ launchers

@@ -227,12 +227,29 @@ int observe(lbm_solver* s, bool with_f) {
   return LBM_OK;
 }
 
-template <class T>
-void depad(const lbm_solver* s, const T* padded, T* out, long plane_off) {
-  const int n = s->cs->n, m = s->cs->m;
-  for (int j = 0; j < m; j++)
-    std::memcpy(out + (size_t)j * n, padded + plane_off + (size_t)(j + 1) * s->pitch + 1,
-                sizeof(T) * n);
+// The real cells of `count` padded planes to the host: put(j, i, w, src,
+// stride) receives cells i .. i + w - 1 of lattice row j, plane k's at
+// src[k * stride].  Several threads call it, for disjoint cells.
+template <class Put>
+int planes_to_host(lbm_solver* s, const double* const* dev, int count, const Put& put) {
+  const size_t n = (size_t)s->cs->n, m = (size_t)s->cs->m, pitch = (size_t)s->pitch;
+  HC(s->staging.to_host(
+      s->stream, (m - 1) * pitch + n, sizeof(double) * (size_t)count,
+      [&](size_t off, size_t len, char* slot) {
+        const void* from[Staging::MAX_PARTS];
+        for (int k = 0; k < count; k++) from[k] = dev[k] + pitch + 1 + off;
+        return s->staging.copy(slot, from, count, sizeof(double) * len, s->stream);
+      },
+      [&](size_t off, size_t len, char* slot) {
+        const double* src = (const double*)slot;
+        for (size_t q = off; q < off + len;) {
+          const size_t j = q / pitch, i = q % pitch;
+          const size_t w = std::min(off + len, j * pitch + n) - q;
+          if (i < n) put(j, i, w, src + (q - off), len);
+          q = (j + 1) * pitch;
+        }
+      }));
+  return LBM_OK;
 }
 
 }  // namespace
@@ -1948,16 +1965,24 @@ int lbm_solver_get_macro(lbm_solver* s, double* rho, double* u, double* v) {
   }
   int rc = observe(s, false);
   if (rc) return rc;
-  std::vector<double> tmp((size_t)s->plane);
   double* outs[3] = {rho, u, v};
-  double* dev[3] = {s->d_rho, s->d_u, s->d_v};
-  for (int a = 0; a < 3; a++) {
-    if (!outs[a]) continue;
-    HC(hipMemcpyAsync(tmp.data(), dev[a], sizeof(double) * s->plane, hipMemcpyDeviceToHost, s->stream));
-    HC(hipStreamSynchronize(s->stream));
-    depad(s, tmp.data(), outs[a], 0);
-  }
-  return LBM_OK;
+  const double* planes[3] = {s->d_rho, s->d_u, s->d_v};
+  double* to[3];
+  const double* from[3];
+  int count = 0;
+  for (int a = 0; a < 3; a++)
+    if (outs[a]) {
+      to[count] = outs[a];
+      from[count++] = planes[a];
+    }
+  if (!count) return LBM_OK;
+  const size_t n = (size_t)s->cs->n;
+  return planes_to_host(s, from, count,
+                        [&](size_t j, size_t i, size_t w, const double* src, size_t stride) {
+                          for (int a = 0; a < count; a++)
+                            std::memcpy(to[a] + j * n + i, src + (size_t)a * stride,
+                                        sizeof(double) * w);
+                        });
 }
 
 int lbm_solver_get_f(lbm_solver* s, double* f, double* metaf) {
@@ -1993,17 +2018,21 @@ int lbm_solver_get_f(lbm_solver* s, double* f, double* metaf) {
   }
   int rc = observe(s, true);
   if (rc) return rc;
-  std::vector<double> tmp((size_t)9 * s->plane), plane_out((size_t)nc);
   double* outs[2] = {f, metaf};
-  double* dev[2] = {s->d_f, s->d_metaf};
+  const double* dev[2] = {s->d_f, s->d_metaf};
   for (int a = 0; a < 2; a++) {
     if (!outs[a]) continue;
-    HC(hipMemcpyAsync(tmp.data(), dev[a], sizeof(double) * 9 * (size_t)s->plane, hipMemcpyDeviceToHost, s->stream));
-    HC(hipStreamSynchronize(s->stream));
-    for (int k = 0; k < 9; k++) {
-      depad(s, tmp.data(), plane_out.data(), (long)k * s->plane);
-      for (long i = 0; i < nc; i++) outs[a][i * 9 + k] = c->fluid[i] == 1 ? plane_out[i] : 0.0;
-    }
+    const double* from[9];
+    for (int k = 0; k < 9; k++) from[k] = dev[a] + (size_t)k * s->plane;
+    rc = planes_to_host(s, from, 9,
+                        [&](size_t j, size_t i, size_t w, const double* src, size_t stride) {
+                          const size_t cell = j * (size_t)c->n + i;
+                          for (size_t x = 0; x < w; x++)
+                            for (size_t k = 0; k < 9; k++)
+                              outs[a][(cell + x) * 9 + k] =
+                                  c->fluid[cell + x] == 1 ? src[k * stride + x] : 0.0;
+                        });
+    if (rc) return rc;
   }
   return LBM_OK;
 }
