@@ -62,7 +62,7 @@ struct lbm_net {
   std::vector<Conv> conv;
   size_t nparam = 0, head_w = 0, head_b = 0;
   float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;  // FP32 master, grad, Adam
-  u16 *pb = nullptr, *wt = nullptr;  // bf16 weights, flipped weights (same offsets)
+  u16 *wf = nullptr, *wt = nullptr;  // packed BF16 weights: convs, data gradients (same offsets)
   int step = 0;
   std::vector<int> Hl, Wl;
   // activations [level], gradients
@@ -193,7 +193,7 @@ int lbm_net_create(int H, int W, int batch, int base, int levels, int in_channel
   if (!rc) rc = nalloc_t(n, &n->g, off);
   if (!rc) rc = nalloc_t(n, &n->m, off);
   if (!rc) rc = nalloc_t(n, &n->v, off);
-  if (!rc) rc = nalloc_t(n, &n->pb, off);
+  if (!rc) rc = nalloc_t(n, &n->wf, off);
   if (!rc) rc = nalloc_t(n, &n->wt, off);
   const int B = batch;
   n->a.assign(L, nullptr);
@@ -333,8 +333,8 @@ static int order(hipStream_t first, hipStream_t later, hipEvent_t ev) {
 }
 
 static int refresh_weights(lbm_net* n) {
-  NC(to_bf16(n->p, n->pb, (long)n->nparam, n->st));
-  for (const Conv& c : n->conv) NC(flip_w(n->pb + c.w, n->wt + c.w, c.Cout, c.C0 + c.C1, n->st));
+  for (const Conv& c : n->conv)
+    NC(pack_w(n->p + c.w, n->wf + c.w, n->wt + c.w, c.Cout, c.C0 + c.C1, n->st));
   return LBM_OK;
 }
 
@@ -365,9 +365,9 @@ static int forward(lbm_net* n, int B) {
   for (int l = 0; l < L; l++) {
     const Conv& ca = n->conv[ci++];
     const Conv& cb = n->conv[ci++];
-    NC(conv3x3(src1(n, x, Cx, l, B, ca.dil), n->pb + ca.w, n->p + ca.b, n->a[l], ca.Cout, true,
+    NC(conv3x3(src1(n, x, Cx, l, B, ca.dil), n->wf + ca.w, n->p + ca.b, nullptr, n->a[l], ca.Cout, true,
                n->st));
-    NC(conv3x3(src1(n, n->a[l], C_of(n, l), l, B, cb.dil), n->pb + cb.w, n->p + cb.b, n->s[l],
+    NC(conv3x3(src1(n, n->a[l], C_of(n, l), l, B, cb.dil), n->wf + cb.w, n->p + cb.b, nullptr, n->s[l],
                cb.Cout, true, n->st));
     if (l < L - 1) {
       NC(pool(n->s[l], n->xp[l], B, n->Hl[l], n->Wl[l], C_of(n, l), n->st));
@@ -382,8 +382,8 @@ static int forward(lbm_net* n, int B) {
     ConvSrc s = src1(n, n->s[l], C_of(n, l), l, B);
     s.in1 = prev;
     s.C1 = C_of(n, l + 1);
-    NC(conv3x3(s, n->pb + ca.w, n->p + ca.b, n->da[l], ca.Cout, true, n->st));
-    NC(conv3x3(src1(n, n->da[l], C_of(n, l), l, B), n->pb + cb.w, n->p + cb.b, n->dd[l], cb.Cout,
+    NC(conv3x3(s, n->wf + ca.w, n->p + ca.b, nullptr, n->da[l], ca.Cout, true, n->st));
+    NC(conv3x3(src1(n, n->da[l], C_of(n, l), l, B), n->wf + cb.w, n->p + cb.b, nullptr, n->dd[l], cb.Cout,
                true, n->st));
     prev = n->dd[l];
   }
@@ -409,9 +409,11 @@ static int conv_grads(lbm_net* n, const Conv& c, const ConvSrc& s, const u16* go
   return LBM_OK;
 }
 
-// data gradient of conv c: gin = conv(gout, flipped W), Cin channels
-static int conv_dgrad(lbm_net* n, const Conv& c, const u16* gout, int l, int B, u16* gin) {
-  return check_hip(conv3x3(src1(n, gout, c.Cout, l, B, c.dil), n->wt + c.w, nullptr, gin,
+// data gradient of conv c: gin = conv(gout, flipped W), Cin channels; with
+// relu_of, the ReLU output that gin is the gradient of, also that ReLU's backward
+static int conv_dgrad(lbm_net* n, const Conv& c, const u16* gout, int l, int B, u16* gin,
+                      const u16* relu_of) {
+  return check_hip(conv3x3(src1(n, gout, c.Cout, l, B, c.dil), n->wt + c.w, nullptr, relu_of, gin,
                            c.C0 + c.C1, false, n->st),
                    "conv dgrad");
 }
@@ -438,9 +440,8 @@ static int backward(lbm_net* n, int B, double fluid, double* loss) {
     const Conv& cb = n->conv[k + 1];
     int rc = conv_grads(n, cb, src1(n, n->da[l], C_of(n, l), l, B), n->gdd[l]);
     if (rc) return rc;
-    rc = conv_dgrad(n, cb, n->gdd[l], l, B, n->gda[l]);
+    rc = conv_dgrad(n, cb, n->gdd[l], l, B, n->gda[l], n->da[l]);
     if (rc) return rc;
-    NC(relu_bwd(n->gda[l], n->da[l], P_of(n, l, B) * C_of(n, l), n->st));
     const u16* prev = (l + 1 <= L - 2) ? n->dd[l + 1] : n->s[L - 1];
     u16* gprev = (l + 1 <= L - 2) ? n->gdd[l + 1] : n->gs[L - 1];
     ConvSrc s = src1(n, n->s[l], C_of(n, l), l, B);
@@ -448,7 +449,7 @@ static int backward(lbm_net* n, int B, double fluid, double* loss) {
     s.C1 = C_of(n, l + 1);
     rc = conv_grads(n, ca, s, n->gda[l]);
     if (rc) return rc;
-    rc = conv_dgrad(n, ca, n->gda[l], l, B, n->dcat[l]);
+    rc = conv_dgrad(n, ca, n->gda[l], l, B, n->dcat[l], nullptr);
     if (rc) return rc;
     NC(up_grad(n->dcat[l], ca.C0 + ca.C1, ca.C0, prev, gprev, B, n->Hl[l], n->Wl[l], ca.C1, n->st));
   }
@@ -461,15 +462,14 @@ static int backward(lbm_net* n, int B, double fluid, double* loss) {
                    n->Hl[l], n->Wl[l], C_of(n, l), n->st));
     int rc = conv_grads(n, cb, src1(n, n->a[l], C_of(n, l), l, B, cb.dil), n->gs[l]);
     if (rc) return rc;
-    rc = conv_dgrad(n, cb, n->gs[l], l, B, n->ga[l]);
+    rc = conv_dgrad(n, cb, n->gs[l], l, B, n->ga[l], n->a[l]);
     if (rc) return rc;
-    NC(relu_bwd(n->ga[l], n->a[l], P_of(n, l, B) * C_of(n, l), n->st));
     const u16* xin = l == 0 ? n->x0 : n->xp[l - 1];
     const int Cx = l == 0 ? CIN0 : C_of(n, l - 1);
     rc = conv_grads(n, ca, src1(n, xin, Cx, l, B, ca.dil), n->ga[l]);
     if (rc) return rc;
     if (l > 0) {
-      rc = conv_dgrad(n, ca, n->ga[l], l, B, n->gxp[l - 1]);
+      rc = conv_dgrad(n, ca, n->ga[l], l, B, n->gxp[l - 1], nullptr);
       if (rc) return rc;
     }
   }
@@ -611,9 +611,10 @@ int lbm_net_train(lbm_net* n, const int* idx, int nb, float lr, double* loss) {
   n->step++;
   const float b1 = 0.9f, b2 = 0.999f;
   const float c1 = 1.0f - std::pow(b1, (float)n->step), c2 = 1.0f - std::pow(b2, (float)n->step);
-  NC(adam(n->p, n->g, n->m, n->v, n->pb, (long)n->nparam, lr, b1, b2, 1e-8f, c1, c2, n->wd,
+  NC(adam(n->p, n->g, n->m, n->v, (long)n->nparam, lr, b1, b2, 1e-8f, c1, c2, n->wd,
           n->st));
-  for (const Conv& c : n->conv) NC(flip_w(n->pb + c.w, n->wt + c.w, c.Cout, c.C0 + c.C1, n->st));
+  rc = refresh_weights(n);
+  if (rc) return rc;
   if (!loss) NC(hipStreamSynchronize(n->st));
   return LBM_OK;
 }

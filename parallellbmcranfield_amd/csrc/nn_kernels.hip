@@ -17,11 +17,14 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "nn_launch.hpp"
 
 namespace lbmnn {
 
 typedef __bf16 bf16;
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -33,6 +36,9 @@ struct Src {  // virtual concat input
   int B, H, W;      // full size
   int dil;          // tap spacing (dilation) of the 3x3 stencil
 };
+
+__device__ inline bf16x8 ld8(const bf16* p) { return *reinterpret_cast<const bf16x8*>(p); }
+__device__ inline void st8(bf16* p, const bf16x8 v) { *reinterpret_cast<bf16x8*>(p) = v; }
 
 __device__ inline bf16x8 zero8() {
   bf16x8 z;
@@ -116,6 +122,7 @@ constexpr int CV_LD = 40;  // LDS row of a weight tile (bf16): 80-byte rows, 16-
 template <int TM, int TN, bool RELU>
 __global__ __launch_bounds__(256) void k_conv3x3(Src s, const bf16* __restrict__ w,
                                                   const float* __restrict__ bias,
+                                                  const bf16* __restrict__ mask,
                                                   bf16* __restrict__ out, int Cout, int nwork) {
   __shared__ __attribute__((aligned(16))) bf16 sw[2][16 * TN][CV_LD];
   const unsigned item = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
@@ -139,11 +146,12 @@ __global__ __launch_bounds__(256) void k_conv3x3(Src s, const bf16* __restrict__
     py[g] = q % s.H;
     pbb[g] = q / s.H;
   }
-  // cooperative weight loader: thread t < 64 TN loads row t / 4 (output
-  // channel cb + t / 4), channels 8 (t % 4) .. + 7 of the K step
-  const int wl_row = threadIdx.x >> 2, wl_col = (threadIdx.x & 3) * 8;
+  // cooperative weight loader: thread t < 64 TN loads what lane t % 64 of the
+  // packed block t / 64 of 16 output channels holds
+  const int wl_row = (threadIdx.x >> 6) * 16 + (threadIdx.x & 15);
+  const int wl_col = ((threadIdx.x >> 4) & 3) * 8;
   const bool wl = threadIdx.x < 64 * TN;
-  const bf16* wsrc = w + (size_t)(cb + (wl ? wl_row : 0)) * 9 * Cin + wl_col;
+  const bf16* wsrc = w + (size_t)(cb + (wl ? wl_row & ~15 : 0)) * 9 * Cin + (threadIdx.x & 63) * 8;
   f32x4 acc[TM][TN];
 #pragma unroll
   for (int g = 0; g < TM; g++)
@@ -183,7 +191,8 @@ __global__ __launch_bounds__(256) void k_conv3x3(Src s, const bf16* __restrict__
       else
         A[g] = *reinterpret_cast<const bf16x8*>(s.in1 + (toff1[g] + (unsigned)(lci - s.C0)));
     }
-    if (wl) wreg = *reinterpret_cast<const bf16x8*>(wsrc + (size_t)lt * Cin + lci);
+    if (wl) wreg = ld8(wsrc);
+    wsrc += 512;
     lci += 32;
     if (lci == Cin) {
       lci = 0;
@@ -234,8 +243,183 @@ __global__ __launch_bounds__(256) void k_conv3x3(Src s, const bf16* __restrict__
         if (p >= P) continue;
         float v = acc[g][h][i] + bv;
         if (RELU) v = v > 0.0f ? v : 0.0f;
-        out[(size_t)p * Cout + co] = (__bf16)v;
+        const size_t o = (size_t)p * Cout + co;
+        if (mask && !((float)mask[o] > 0.0f)) v = 0.0f;
+        out[o] = (__bf16)v;
       }
+  }
+}
+
+// ------------------------------------------------------------ conv, tiles in LDS
+// The same sums as k_conv3x3 (K in the same order: tap, then blocks of 32
+// channels, so the same bits), from a tile of tw x th output pixels whose
+// input, with its halo, is staged in LDS once: k_conv3x3 fetches every pixel
+// nine times through the vector cache (64 bytes per clock), and its K loop
+// meets a barrier each step.  Here the K loop has no barrier: pixels come from
+// LDS (a tap is an offset; pixels outside the image are staged as zeros),
+// weights straight from memory (the waves of a workgroup read the same
+// kilobytes, which the vector cache serves), both one step ahead of the MFMAs.
+// What bounds it: the vector cache and the LDS, each about as long as the
+// MFMAs at 64 pixels x 32 channels per wave; at 32 channels the memory.
+// 16 x 257 x 257: 32 -> 32 channels 85 -> 42 us (135 MB), 96 -> 32
+// 186 -> 119, 32 -> 96 231 -> 113; 16 x 129 x 129: 64 -> 64 84 -> 34 (580
+// TFLOP/s), 192 -> 64 169 -> 93; 16 x 65 x 65: 128 -> 128 60 -> 32,
+// 384 -> 128 130 -> 88; 16 x 33 x 33 dilated by 4: 128 -> 256 39 -> 24.
+// 128 pixels or 64 channels per wave were 10-50 % slower (fewer waves), and
+// weights two steps ahead up to 35 %.
+// A workgroup is pw x cw waves: pixel groups of 64 of the tile, flattened
+// row by row, by channel blocks of 32; a wave takes blocks cw apart, so the
+// staged pixels serve all Cout.  The weights are the MFMA's rows and the
+// pixels its columns: a lane ends with four consecutive channels of one pixel,
+// one 8-byte store each.  ReLU, or for a data gradient the ReLU mask of the
+// tensor that the gradient belongs to (zero where that is not above zero), is
+// applied to the value as it is stored.
+// One image tile per workgroup; the grid deals contiguous runs of tiles to
+// the XCDs as k_conv3x3 does, so a tile's halo is its neighbours' pixels in
+// the same L2.
+constexpr int CT_TM = 4, CT_TN = 2;  // 16 x 16 tiles of a wave: pixels by output channels
+struct ConvTile {
+  int tw, th, nx, ny;  // tile size; tiles per row and column of an image
+  int pw, cw;          // waves over pixels and over channel blocks
+  unsigned inv_g, inv_row, inv_tw;  // ceil(2^32 / d): q / d = umulhi(q, inv) for q d < 2^32
+};
+
+template <bool RELU>
+__global__ __launch_bounds__(512) void k_conv_tile(Src s, const bf16* __restrict__ w,
+                                                   const float* __restrict__ bias,
+                                                   const bf16* __restrict__ mask,
+                                                   bf16* __restrict__ out, int Cout, ConvTile ct,
+                                                   int nwork) {
+  extern __shared__ __attribute__((aligned(16))) bf16 sx[];  // [halo pixel][Cin + 8]
+  constexpr int TM = CT_TM, TN = CT_TN, STAGE = 6;
+  const unsigned item = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (item >= (unsigned)nwork) return;
+  const int per = ct.nx * ct.ny;
+  const int b = (int)item / per, ti = (int)item % per;
+  const int y0 = ti / ct.nx * ct.th, x0 = ti % ct.nx * ct.tw;
+  const int Cin = s.C0 + s.C1, ld = Cin + 8;
+  const int row = ct.tw + 2 * s.dil, npx = row * (ct.th + 2 * s.dil);
+  const int nthr = (int)blockDim.x;
+
+  const int G = Cin / 8, total = npx * G;
+  const int Hc = (s.H + 1) >> 1, Wc = (s.W + 1) >> 1;
+  for (int i0 = (int)threadIdx.x; i0 < total; i0 += nthr * STAGE) {
+    bf16x8 v[STAGE];
+    int at[STAGE];
+#pragma unroll
+    for (int k = 0; k < STAGE; k++) {
+      const int i = i0 + k * nthr;
+      const int q = (int)__umulhi((unsigned)i, ct.inv_g), c = (i - q * G) * 8;
+      const int qy = (int)__umulhi((unsigned)q, ct.inv_row);
+      const int y = y0 - s.dil + qy, x = x0 - s.dil + (q - qy * row);
+      at[k] = q * ld + c;
+      v[k] = zero8();
+      if (i < total && y >= 0 && y < s.H && x >= 0 && x < s.W)
+        v[k] = c < s.C0
+                   ? ld8(s.in0 + ((unsigned)(b * s.H + y) * (unsigned)s.W + (unsigned)x) *
+                                     (unsigned)s.C0 + (unsigned)c)
+                   : ld8(s.in1 + ((unsigned)(b * Hc + (y >> 1)) * (unsigned)Wc +
+                                  (unsigned)(x >> 1)) * (unsigned)s.C1 + (unsigned)(c - s.C0));
+    }
+#pragma unroll
+    for (int k = 0; k < STAGE; k++)
+      if (i0 + k * nthr < total) st8(sx + at[k], v[k]);
+  }
+  __syncthreads();
+
+  const int wave = (int)threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int r = lane & 15, kb = lane >> 4;
+  const int wp = wave % ct.pw, wc = wave / ct.pw;
+  int base[TM];       // LDS offset of the lane's pixel at tap 0
+  unsigned pix[TM];   // its index in the image batch
+  bool ok[TM];
+#pragma unroll
+  for (int g = 0; g < TM; g++) {
+    const int q = (wp * TM + g) * 16 + r;
+    const int ty = (int)__umulhi((unsigned)q, ct.inv_tw), tx = q - ty * ct.tw;
+    ok[g] = ty < ct.th && y0 + ty < s.H && x0 + tx < s.W;
+    base[g] = (ok[g] ? (ty * row + tx) * ld : 0) + kb * 8;
+    pix[g] = (unsigned)(b * s.H + y0 + ty) * (unsigned)s.W + (unsigned)(x0 + tx);
+  }
+  const int nc = Cin / 32, nk = 9 * nc;
+  for (int cblk = wc; cblk * 16 * TN < Cout; cblk += ct.cw) {
+    const int cb = cblk * 16 * TN;
+    const bf16* wp0 = w + (size_t)cb * 9 * Cin + lane * 8;
+    const unsigned wblk = 16u * 9u * (unsigned)Cin;  // to the next 16 output channels
+    f32x4 acc[TM][TN];
+#pragma unroll
+    for (int g = 0; g < TM; g++)
+#pragma unroll
+      for (int h = 0; h < TN; h++) acc[g][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+    int lc = 0, lx = 0, off = 0;  // LDS offset of the next step's pixels
+    unsigned wo = 0;              // offset of the next step's weights
+    auto load_a = [&](bf16x8 (&A)[TM]) {
+#pragma unroll
+      for (int g = 0; g < TM; g++) A[g] = ld8(sx + base[g] + off);
+      off += 32;
+      if (++lc == nc) {  // next tap
+        lc = 0;
+        off += s.dil * ld - Cin;
+        if (++lx == 3) {
+          lx = 0;
+          off += s.dil * (row - 3) * ld;
+        }
+      }
+    };
+    auto load_b = [&](bf16x8 (&Bm)[TN]) {
+#pragma unroll
+      for (int h = 0; h < TN; h++) Bm[h] = ld8(wp0 + (wo + (unsigned)h * wblk));
+      wo += 512;
+    };
+    auto mma = [&](const bf16x8 (&A)[TM], const bf16x8 (&Bm)[TN]) {
+#pragma unroll
+      for (int g = 0; g < TM; g++)
+#pragma unroll
+        for (int h = 0; h < TN; h++)
+          acc[g][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Bm[h], A[g], acc[g][h], 0, 0, 0);
+    };
+    bf16x8 a0[TM], a1[TM], b0[TN], b1[TN];
+    load_b(b0);
+    load_a(a0);
+    for (int kk = 0;;) {
+      if (kk + 1 < nk) {
+        load_b(b1);
+        load_a(a1);
+      }
+      mma(a0, b0);
+      if (++kk == nk) break;
+      if (kk + 1 < nk) {
+        load_b(b0);
+        load_a(a0);
+      }
+      mma(a1, b1);
+      if (++kk == nk) break;
+    }
+#pragma unroll
+    for (int h = 0; h < TN; h++) {
+      const int co = cb + h * 16 + kb * 4;
+      f32x4 bv = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (bias) bv = *reinterpret_cast<const f32x4*>(bias + co);
+#pragma unroll
+      for (int g = 0; g < TM; g++) {
+        if (!ok[g]) continue;
+        const size_t o = (size_t)pix[g] * (unsigned)Cout + (unsigned)co;
+        bf16x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          float f = acc[g][h][i] + bv[i];
+          if (RELU) f = f > 0.0f ? f : 0.0f;
+          v[i] = (__bf16)f;
+        }
+        if (mask) {
+          const bf16x4 y = *reinterpret_cast<const bf16x4*>(mask + o);
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            if (!((float)y[i] > 0.0f)) v[i] = (__bf16)0.0f;
+        }
+        *reinterpret_cast<bf16x4*>(out + o) = v;
+      }
+    }
   }
 }
 
@@ -288,7 +472,6 @@ __device__ inline bool wgrad_item(int T, int Cout, int Cin, int nwork, WgItem& w
 
 constexpr int WG_PX = 64;          // pixels per K step of a wave
 constexpr int WG_LD = WG_PX + 8;   // LDS row (bf16): 144-byte rows keep 16-byte reads aligned
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 __global__ __launch_bounds__(256) void k_wgrad(Src s, const bf16* __restrict__ dout, int Cout,
                                                float* __restrict__ part, int grp_per_chunk,
                                                int nwork) {
@@ -564,33 +747,31 @@ __global__ __launch_bounds__(256) void k_reduce_chunks(const float* __restrict__
 }
 
 // ------------------------------------------------------------ elementwise
-// w'[ci][t][co] = w[co][8 - t][ci]: the data-gradient conv's weights.
-__global__ void k_flip_w(const bf16* __restrict__ w, bf16* __restrict__ wt, int Cout, int Cin) {
+// A conv's weights in the order that the MFMAs read them: for each block of
+// 16 output channels and each K step (tap, block of 32 input channels), the
+// 64 lanes' 16 bytes one after the other, lane 16 kb + r holding channels
+// 8 kb .. + 7 of output channel r.  A wave's operand is then one contiguous
+// kilobyte: as rows of [co][tap][ci] it was 16 pieces of 64 bytes, which the
+// vector cache hands out at half the rate (the 64-to-64-channel conv at
+// 16 x 129 x 129 took 66 us from rows, 34 us so).
+__device__ inline size_t packed_w(int co, int t, int ci, int Cin) {
+  return (((size_t)(co >> 4) * 9 + t) * (Cin >> 5) + (ci >> 5)) * 512 +
+         (((ci >> 3) & 3) * 16 + (co & 15)) * 8 + (ci & 7);
+}
+
+// BF16 weights of a conv and of its data gradient, w'[ci][t][co] =
+// w[co][8 - t][ci], both packed, from the FP32 [Cout][9][Cin].
+__global__ void k_pack_w(const float* __restrict__ w, bf16* __restrict__ wf,
+                         bf16* __restrict__ wt, int Cout, int Cin) {
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
   const long n = (long)Cout * 9 * Cin;
   if (i >= n) return;
   const int ci = (int)(i % Cin);
   const int t = (int)((i / Cin) % 9);
   const int co = (int)(i / (9L * Cin));
-  wt[((size_t)ci * 9 + (8 - t)) * Cout + co] = w[i];
-}
-
-__global__ void k_to_bf16(const float* __restrict__ a, bf16* __restrict__ b, long n) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) b[i] = (__bf16)a[i];
-}
-
-// g *= (y > 0) (ReLU backward; y is the stored post-activation output).
-// g[i] = 0 where y[i] <= 0; eight elements per thread (n % 8 == 0, 16-byte
-// aligned buffers: the host checks)
-__global__ void k_relu_bwd(bf16* __restrict__ g, const bf16* __restrict__ y, long n8) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n8) return;
-  const bf16x8 yv = reinterpret_cast<const bf16x8*>(y)[i];
-  bf16x8 gv = reinterpret_cast<const bf16x8*>(g)[i];
-  for (int e = 0; e < 8; e++)
-    if (!((float)yv[e] > 0.0f)) gv[e] = (__bf16)0.0f;
-  reinterpret_cast<bf16x8*>(g)[i] = gv;
+  const bf16 v = (__bf16)w[i];
+  wf[packed_w(co, t, ci, Cin)] = v;
+  wt[packed_w(ci, 8 - t, co, Cout)] = v;
 }
 
 // Eight consecutive channels as floats, and back.
@@ -604,8 +785,6 @@ __device__ inline bf16x8 pack8(const float* f) {
   for (int e = 0; e < 8; e++) v[e] = (__bf16)f[e];
   return v;
 }
-__device__ inline bf16x8 ld8(const bf16* p) { return *reinterpret_cast<const bf16x8*>(p); }
-__device__ inline void st8(bf16* p, const bf16x8 v) { *reinterpret_cast<bf16x8*>(p) = v; }
 
 // The elementwise kernels below take eight consecutive channels per thread
 // (16-byte accesses; every channel count is a multiple of 8 and the element
@@ -857,8 +1036,8 @@ __global__ __launch_bounds__(256) void k_head_wgrad_part(const float* __restrict
 // ------------------------------------------------------------ optimiser
 // Adam on the FP32 master copy; bf16 copy of the same element refreshed.
 __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, bf16* __restrict__ pb, long n, float lr, float b1,
-                       float b2, float eps, float c1, float c2, float wd) {
+                       float* __restrict__ v, long n, float lr, float b1, float b2, float eps,
+                       float c1, float c2, float wd) {
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
   const float gi = g[i];
@@ -867,9 +1046,7 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float
   m[i] = mi;
   v[i] = vi;
   const float upd = lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-  const float np = p[i] - upd - lr * wd * p[i];  // decoupled weight decay (AdamW)
-  p[i] = np;
-  pb[i] = (__bf16)np;
+  p[i] = p[i] - upd - lr * wd * p[i];  // decoupled weight decay (AdamW)
 }
 
 // ------------------------------------------------------------ data
@@ -906,29 +1083,90 @@ static inline Src src_of(const ConvSrc& c) {
 }
 
 template <int TM, int TN>
-static void launch_conv(const Src& s, const u16* w, const float* bias, u16* out, int Cout,
-                        long P, bool relu, hipStream_t st) {
+static void launch_conv(const Src& s, const u16* w, const float* bias, const u16* mask, u16* out,
+                        int Cout, long P, bool relu, hipStream_t st) {
   const long nwork = (P + 64 * TM - 1) / (64 * TM) * (Cout / (16 * TN));
   const unsigned g = (unsigned)((nwork + 7) / 8 * 8);  // a multiple of 8 (k_conv3x3)
-  if (relu) k_conv3x3<TM, TN, true><<<g, 256, 0, st>>>(s, cb(w), bias, mb(out), Cout, (int)nwork);
-  else k_conv3x3<TM, TN, false><<<g, 256, 0, st>>>(s, cb(w), bias, mb(out), Cout, (int)nwork);
+  if (relu)
+    k_conv3x3<TM, TN, true><<<g, 256, 0, st>>>(s, cb(w), bias, cb(mask), mb(out), Cout, (int)nwork);
+  else
+    k_conv3x3<TM, TN, false><<<g, 256, 0, st>>>(s, cb(w), bias, cb(mask), mb(out), Cout, (int)nwork);
 }
 
-// Tile choice: 64 output channels per wave where Cout allows, 64 pixels per
-// wave while that still gives >= 1024 workgroups (4 per CU), else 32.
-hipError_t conv3x3(const ConvSrc& cs, const u16* w, const float* bias, u16* out, int Cout,
-                   bool relu, hipStream_t st) {
+static inline unsigned inv32(int d) { return (unsigned)(((1ULL << 32) + d - 1) / d); }
+
+// The tile of a conv: for 4, 2 and 1 waves over pixels, every width whose
+// rows fill the tile, at the least cost that the busiest of the 256 CUs has,
+// in its clocks: MFMAs (all pixels of a tile, the unused ones too) and the
+// staged bytes at the 16 per clock that a CU gets from the L2.  False where no
+// tile fits the LDS (dilated or deep convs).
+static bool tile_plan(const Src& s, int Cout, ConvTile& best, int& best_lds, long& nwork) {
+  constexpr int LDS_MAX = 160 << 10, CUS = 256;
+  const int Cin = s.C0 + s.C1, nblocks = Cout / (16 * CT_TN);
+  long best_cost = 0;
+  bool found = false;
+  for (int pw = 4; pw >= 1; pw /= 2) {
+    const int px = 16 * CT_TM * pw;
+    for (int w = 8; w <= 64; w++) {
+      ConvTile t{};
+      t.nx = (s.W + w - 1) / w;
+      t.tw = (s.W + t.nx - 1) / t.nx;
+      if (t.tw < 2) continue;  // inv_tw holds divisors of at least 2
+      t.th = std::min(s.H, px / t.tw);
+      t.ny = (s.H + t.th - 1) / t.th;
+      t.th = (s.H + t.ny - 1) / t.ny;
+      const int row = t.tw + 2 * s.dil;
+      const long lds = (long)row * (t.th + 2 * s.dil) * (Cin + 8) * 2;
+      if (lds > LDS_MAX) continue;
+      const long n = (long)s.B * t.nx * t.ny;
+      const long cost = (n + CUS - 1) / CUS * ((long)px * Cout * Cin * 9 / 2048 + lds / 16);
+      if (found && cost >= best_cost) continue;
+      found = true;
+      best_cost = cost;
+      t.pw = pw;
+      t.cw = 1;
+      while (t.cw < 8 / pw && 2 * t.cw <= nblocks) t.cw *= 2;
+      t.inv_g = inv32(Cin / 8);
+      t.inv_row = inv32(row);
+      t.inv_tw = inv32(t.tw);
+      best = t;
+      best_lds = (int)lds;
+      nwork = n;
+    }
+  }
+  return found;
+}
+
+// k_conv3x3 where no tile fits the LDS (8 x 1 pixels with a halo of 8 need
+// 215 kB at 256 channels): 64 output channels per wave where Cout allows, 64 pixels
+// per wave while that still gives >= 1024 workgroups (4 per CU), else 32.
+hipError_t conv3x3(const ConvSrc& cs, const u16* w, const float* bias, const u16* mask, u16* out,
+                   int Cout, bool relu, hipStream_t st) {
   const Src s = src_of(cs);
   const long P = (long)cs.B * cs.H * cs.W;
-  if (Cout % 32 || (cs.C0 + cs.C1) % 32 || P + 256 > 0x7fffffffL) return hipErrorInvalidValue;
+  if (Cout % 32 || (cs.C0 + cs.C1) % 32 || P + 256 > 0x7fffffffL ||
+      (reinterpret_cast<uintptr_t>(bias) & 15))
+    return hipErrorInvalidValue;
+  ConvTile t;
+  int lds;
+  long nwork;
+  if (tile_plan(s, Cout, t, lds, nwork)) {
+    const unsigned g = (unsigned)((nwork + 7) / 8 * 8);  // a multiple of 8, as above
+    const int nthr = 64 * t.pw * t.cw;
+    if (relu)
+      k_conv_tile<true><<<g, nthr, lds, st>>>(s, cb(w), bias, cb(mask), mb(out), Cout, t, (int)nwork);
+    else
+      k_conv_tile<false><<<g, nthr, lds, st>>>(s, cb(w), bias, cb(mask), mb(out), Cout, t, (int)nwork);
+    return hipGetLastError();
+  }
   const int TN = Cout % 64 == 0 ? 4 : 2;
   const long wg4 = (P + 255) / 256 * (Cout / (16 * TN));
   if (TN == 4) {
-    if (wg4 >= 1024) launch_conv<4, 4>(s, w, bias, out, Cout, P, relu, st);
-    else launch_conv<2, 4>(s, w, bias, out, Cout, P, relu, st);
+    if (wg4 >= 1024) launch_conv<4, 4>(s, w, bias, mask, out, Cout, P, relu, st);
+    else launch_conv<2, 4>(s, w, bias, mask, out, Cout, P, relu, st);
   } else {
-    if (wg4 >= 1024) launch_conv<4, 2>(s, w, bias, out, Cout, P, relu, st);
-    else launch_conv<2, 2>(s, w, bias, out, Cout, P, relu, st);
+    if (wg4 >= 1024) launch_conv<4, 2>(s, w, bias, mask, out, Cout, P, relu, st);
+    else launch_conv<2, 2>(s, w, bias, mask, out, Cout, P, relu, st);
   }
   return hipGetLastError();
 }
@@ -970,20 +1208,9 @@ hipError_t reduce_chunks(const float* part, int nchunk, long n, float* out, hipS
   return hipGetLastError();
 }
 
-hipError_t flip_w(const u16* w, u16* wt, int Cout, int Cin, hipStream_t st) {
-  k_flip_w<<<nblk((long)Cout * 9 * Cin), 256, 0, st>>>(cb(w), mb(wt), Cout, Cin);
-  return hipGetLastError();
-}
-
-hipError_t to_bf16(const float* a, u16* b, long n, hipStream_t st) {
-  k_to_bf16<<<nblk(n), 256, 0, st>>>(a, mb(b), n);
-  return hipGetLastError();
-}
-
-hipError_t relu_bwd(u16* g, const u16* y, long n, hipStream_t st) {
-  if (n % 8 || ((reinterpret_cast<uintptr_t>(g) | reinterpret_cast<uintptr_t>(y)) & 15))
-    return hipErrorInvalidValue;
-  k_relu_bwd<<<nblk(n / 8), 256, 0, st>>>(mb(g), cb(y), n / 8);
+hipError_t pack_w(const float* w, u16* wf, u16* wt, int Cout, int Cin, hipStream_t st) {
+  if (Cout % 32 || Cin % 32) return hipErrorInvalidValue;
+  k_pack_w<<<nblk((long)Cout * 9 * Cin), 256, 0, st>>>(w, mb(wf), mb(wt), Cout, Cin);
   return hipGetLastError();
 }
 
@@ -1050,9 +1277,9 @@ hipError_t head_wgrad_part(const float* dy, const u16* x, float* part, int P, in
   return hipGetLastError();
 }
 
-hipError_t adam(float* p, const float* g, float* m, float* v, u16* pb, long n, float lr, float b1,
+hipError_t adam(float* p, const float* g, float* m, float* v, long n, float lr, float b1,
                 float b2, float eps, float c1, float c2, float wd, hipStream_t st) {
-  k_adam<<<nblk(n), 256, 0, st>>>(p, g, m, v, mb(pb), n, lr, b1, b2, eps, c1, c2, wd);
+  k_adam<<<nblk(n), 256, 0, st>>>(p, g, m, v, n, lr, b1, b2, eps, c1, c2, wd);
   return hipGetLastError();
 }
 

@@ -20,9 +20,11 @@ struct ConvSrc {
   int dil = 1;  // dilation of the 3x3 stencil
 };
 
-// out = act(conv3x3(src, w) + bias); w is [Cout][9][C0 + C1], bias may be null.
-hipError_t conv3x3(const ConvSrc& s, const u16* w, const float* bias, u16* out, int Cout,
-                   bool relu, hipStream_t st);
+// out = act(conv3x3(src, w) + bias), zero where mask (laid out as out) is not
+// above zero; w is a [Cout][9][C0 + C1] that pack_w packed, bias and mask may
+// be null.
+hipError_t conv3x3(const ConvSrc& s, const u16* w, const float* bias, const u16* mask, u16* out,
+                   int Cout, bool relu, hipStream_t st);
 // Weight-gradient partial sums, one [Cout][9][Cin] block per chunk of
 // grp_per_chunk groups of 64 consecutive pixels (Cout, Cin multiples of 32).
 // (co, ci) tile edge of a workgroup: 64 when both counts are multiples of 64
@@ -33,9 +35,8 @@ hipError_t wgrad(const ConvSrc& s, const u16* dout, int Cout, float* part, int g
                  hipStream_t st);
 hipError_t colsum_part(const u16* g, int P, int C, int px_per_chunk, float* part, hipStream_t st);
 hipError_t reduce_chunks(const float* part, int nchunk, long n, float* out, hipStream_t st);
-hipError_t flip_w(const u16* w, u16* wt, int Cout, int Cin, hipStream_t st);
-hipError_t to_bf16(const float* a, u16* b, long n, hipStream_t st);
-hipError_t relu_bwd(u16* g, const u16* y, long n, hipStream_t st);
+// wf: the BF16 weights of a conv, packed for conv3x3; wt: its data gradient's.
+hipError_t pack_w(const float* w, u16* wf, u16* wt, int Cout, int Cin, hipStream_t st);
 // Divergence penalty of the predicted velocity: d (per pixel) and its
 // per-256-pixel sums of d^2 into part; dy += the gradient of (g / 2) sum d^2.
 hipError_t div_penalty(const float* y, const float* mask, float* d, float* part, float* dy, int B,
@@ -53,8 +54,8 @@ hipError_t head_bwd(const float* dy, const float* w, const u16* x, u16* dx, int 
                     hipStream_t st);
 hipError_t head_wgrad_part(const float* dy, const u16* x, float* part, int P, int C, int K,
                            int px_per_chunk, hipStream_t st);
-hipError_t adam(float* p, const float* g, float* m, float* v, u16* pb, long n, float lr, float b1,
-                float b2, float eps, float c1, float c2, float wd, hipStream_t st);
+hipError_t adam(float* p, const float* g, float* m, float* v, long n, float lr, float b1, float b2,
+                float eps, float c1, float c2, float wd, hipStream_t st);
 hipError_t gather(const float* inputs, const float* targets, const int* idx, u16* x, float* t,
                   float* mask, int B, int HW, int Ci, int Cp, hipStream_t st);
 
