@@ -114,17 +114,6 @@ static ConvSrc src1(const lbm_net* n, const u16* x, int C, int l, int B, int dil
   return s;
 }
 
-// chunking of a conv's weight gradient: about 2048 workgroups per launch
-// (fewer chunks = less partial-sum traffic for the fixed-order reduction)
-static int grp_per_chunk(const lbm_net* n, const Conv& c, const ConvSrc& s) {
-  const long ngrp = wgrad_groups(s);
-  const int T = wgrad_tile(c.Cout, c.C0 + c.C1);
-  const long per = (long)(c.Cout / T) * 9 * ((c.C0 + c.C1) / T);
-  long chunks = std::max(1L, 2048 / per);
-  (void)n;
-  return (int)std::max(1L, (ngrp + chunks - 1) / chunks);
-}
-
 // uniform (0,1] from a 64-bit LCG: deterministic initialisation on every host
 static double urand(uint64_t& st) {
   st = st * 6364136223846793005ULL + 1442695040888963407ULL;
@@ -240,10 +229,12 @@ int lbm_net_create(int H, int W, int batch, int base, int levels, int in_channel
   // bias and head partials
   size_t cap = 0;
   for (const Conv& c : n->conv) {
-    ConvSrc s = src1(n, nullptr, c.C0, c.level, B);
+    ConvSrc s = src1(n, nullptr, c.C0, c.level, B, c.dil);
     s.C1 = c.C1;
-    const int ch = wgrad_chunks(s, grp_per_chunk(n, c, s));
-    cap = std::max(cap, (size_t)ch * c.Cout * 9 * (c.C0 + c.C1));
+    for (int k = 1; k <= B; k++) {  // a smaller batch may have larger tiles' chunks
+      s.B = k;
+      cap = std::max(cap, (size_t)wgrad_plan(s, c.Cout).chunks * c.Cout * (9 * (c.C0 + c.C1) + 1));
+    }
     cap = std::max(cap, (size_t)((P_of(n, c.level, B) + RED_CHUNK - 1) / RED_CHUNK) * c.Cout);
   }
   cap = std::max(cap, (size_t)((P0 + RED_CHUNK - 1) / RED_CHUNK) * (KOUT * base + KOUT));
@@ -394,15 +385,16 @@ static int forward(lbm_net* n, int B) {
 
 // weight + bias gradient of conv c (input s, output gradient gout) into n->g
 static int conv_grads(lbm_net* n, const Conv& c, const ConvSrc& s, const u16* gout) {
-  const int spc = grp_per_chunk(n, c, s);
-  const int ch = wgrad_chunks(s, spc);
-  const long nw = (long)c.Cout * 9 * (c.C0 + c.C1);
-  if ((size_t)ch * nw > n->part_cap) {
+  const WgradPlan plan = wgrad_plan(s, c.Cout);
+  const long nw = (long)c.Cout * 9 * (c.C0 + c.C1);  // c.b is c.w + nw
+  const long row = nw + (plan.with_bias ? c.Cout : 0);
+  if ((size_t)plan.chunks * row > n->part_cap) {
     set_error("network scratch too small");
     return LBM_EINVAL;
   }
-  NC(wgrad(s, gout, c.Cout, n->part, spc, n->st));
-  NC(reduce_chunks(n->part, ch, nw, n->g + c.w, n->st));
+  NC(wgrad(s, gout, c.Cout, n->part, n->st));
+  NC(reduce_chunks(n->part, plan.chunks, row, n->g + c.w, n->st));
+  if (plan.with_bias) return LBM_OK;
   const int P = s.B * s.H * s.W;
   NC(colsum_part(gout, P, c.Cout, RED_CHUNK, n->part, n->st));
   NC(reduce_chunks(n->part, (P + RED_CHUNK - 1) / RED_CHUNK, c.Cout, n->g + c.b, n->st));

@@ -692,6 +692,182 @@ __global__ __launch_bounds__(256) void k_wgrad64(Src s, const bf16* __restrict__
       }
 }
 
+// The same sums from pixel tiles staged in LDS as they are in memory: a
+// workgroup takes a (co, ci) block of all nine taps and, one after the other,
+// the tiles of its chunk.  Of each it stages dout's 16 TCO channels and the
+// input's 16 WCI channels with the halo (zeros outside the image) and
+// multiplies: a tap is an offset into the staged input, so a pixel is fetched
+// once and not per tap, and the LDS's transposing reads (four pixels of 16
+// channels to 16 lanes, four pixels of one channel each) give both operands,
+// so nothing is transposed by hand.  Wave (wci, wk) owns all TCO co tiles by
+// ci tile wci and every WK-th group of 32 pixels; a group's dout operands
+// serve nine taps.  The WK waves' sums are added in LDS at the end.  The bias
+// gradient is one more product, by a column of ones, in the workgroups of the
+// first ci block.  Two workgroups per CU, one staging while one multiplies.
+// Bound by the LDS reads (13 kB per 36 MFMAs with TCO = 4) and at 32 channels
+// by memory.  With the pass for the bias that it saves, against k_wgrad64 and
+// k_wgrad: 64 x 64 channels at 16 x 129 x 129 96 + 18 -> 47 us, 128 x 128 at
+// 16 x 65 x 65 96 + 18 -> 42, 32 x 32 at 16 x 257 x 257 126 + 18 -> 55.
+struct WgTile {
+  int tw, th, nx, ny;  // tile size; tiles per row and column of an image
+  int groups;          // groups of 32 pixels of a tile, a multiple of WK
+  int tiles, per_chunk;
+  unsigned inv_row, inv_tw;  // as ConvTile
+};
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ inline bf16x8 ld_tr(const bf16* p0, const bf16* p1) {
+  typedef __attribute__((address_space(3))) s16x4* lds_ptr;
+  union {
+    s16x4 s[2];
+    bf16x8 v;
+  } u;
+  u.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)p0);
+  u.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)p1);
+  return u.v;
+}
+
+template <int TCO, int WCI, int WK>
+__global__ __launch_bounds__(256, 2) void k_wgrad_tile(Src s, const bf16* __restrict__ dout,
+                                                       int Cout, float* __restrict__ part,
+                                                       WgTile wt, int nwork) {
+  extern __shared__ __attribute__((aligned(16))) bf16 sx[];
+  constexpr int CO = 16 * TCO, CI = 16 * WCI, LDO = CO + 8, LDI = CI + 8, MAXG = 4, STAGE = 6;
+  const unsigned item = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (item >= (unsigned)nwork) return;
+  const int Cin = s.C0 + s.C1, nci = Cin / CI, nco = Cout / CO;
+  const int cib = (int)item % nci * CI, cob = (int)item / nci % nco * CO;
+  const int chunk = (int)item / (nci * nco);
+  const int wave = (int)threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wci = wave % WCI, wk = wave / WCI;
+  const int r = lane & 15, kb = lane >> 4;
+  const int row = wt.tw + 2 * s.dil, npx = row * (wt.th + 2 * s.dil);
+  const int opx = wt.groups * 32;
+  bf16* const so = sx;                       // dout [opx][LDO]
+  bf16* const si = sx + (size_t)opx * LDO;   // input [npx][LDI]
+  const int Hc = (s.H + 1) >> 1, Wc = (s.W + 1) >> 1;
+
+  // the lane's pixels of its wave's groups: four channels 4 (r % 4) .. of
+  // pixels kb * 4 + r / 4 and 16 more, as the transposing read wants them
+  int xin[MAXG][2];
+#pragma unroll
+  for (int g = 0; g < MAXG; g++)
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+      const int q = (g * WK + wk) * 32 + e * 16 + kb * 4 + (r >> 2);
+      const int ty = (int)__umulhi((unsigned)q, wt.inv_tw), tx = q - ty * wt.tw;
+      xin[g][e] = (ty < wt.th ? (ty * row + tx) * LDI : 0) + wci * 16 + (r & 3) * 4;
+    }
+  const int xout = (wk * 32 + kb * 4 + (r >> 2)) * LDO + (r & 3) * 4;
+
+  f32x4 acc[9][TCO], accb[TCO];
+#pragma unroll
+  for (int h = 0; h < TCO; h++) {
+    accb[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < 9; t++) acc[t][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const bool bias = cib == 0 && wci == 0;
+  bf16x8 ones;
+#pragma unroll
+  for (int e = 0; e < 8; e++) ones[e] = (__bf16)1.0f;
+
+  const int t1 = min(wt.tiles, (chunk + 1) * wt.per_chunk);
+  for (int ti = chunk * wt.per_chunk; ti < t1; ti++) {
+    const int per = wt.nx * wt.ny, b = ti / per, tq = ti % per;
+    const int y0 = tq / wt.nx * wt.th, x0 = tq % wt.nx * wt.tw;
+    const int nout = opx * (CO / 8), total = nout + npx * (CI / 8);
+    for (int i0 = (int)threadIdx.x; i0 < total; i0 += 256 * STAGE) {
+      bf16x8 v[STAGE];
+      int at[STAGE];
+      bool ok[STAGE];
+#pragma unroll
+      for (int k = 0; k < STAGE; k++) {
+        const int i = i0 + k * 256;
+        const bool o = i < nout;
+        const int j = o ? i : i - nout;
+        const int q = j / (o ? CO / 8 : CI / 8), c = j % (o ? CO / 8 : CI / 8) * 8;
+        const int qy = (int)__umulhi((unsigned)q, o ? wt.inv_tw : wt.inv_row);
+        const int y = y0 + qy - (o ? 0 : s.dil), x = x0 + q - qy * (o ? wt.tw : row) - (o ? 0 : s.dil);
+        at[k] = o ? q * LDO + c : opx * LDO + q * LDI + c;
+        ok[k] = i < total && y >= 0 && y < s.H && x >= 0 && x < s.W && (!o || qy < wt.th);
+        const bool coarse = !o && cib + c >= s.C0;
+        const int ch = o ? cob + c : cib + c - (coarse ? s.C0 : 0);
+        const unsigned px = coarse ? (unsigned)(b * Hc + (y >> 1)) * (unsigned)Wc + (unsigned)(x >> 1)
+                                   : (unsigned)(b * s.H + y) * (unsigned)s.W + (unsigned)x;
+        const bf16* src = o ? dout : coarse ? s.in1 : s.in0;
+        const unsigned off = px * (unsigned)(o ? Cout : coarse ? s.C1 : s.C0) + (unsigned)ch;
+        v[k] = ld8(src + (ok[k] ? off : 0u));  // outside: any element, not stored
+      }
+#pragma unroll
+      for (int k = 0; k < STAGE; k++)
+        if (i0 + k * 256 < total) st8(sx + at[k], ok[k] ? v[k] : zero8());
+    }
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < MAXG; g++) {
+      if (g * WK >= wt.groups) break;
+      bf16x8 a[TCO], x[3];
+      const bf16* po = so + xout + g * WK * 32 * LDO;
+      int x0 = xin[g][0], x1 = xin[g][1];
+      asm("" : "+v"(x0), "+v"(x1));  // not 72 addresses held across tiles
+      auto tap = [&](int t) {
+        const int off = (t / 3 * row + t % 3) * s.dil * LDI;
+        return ld_tr(si + x0 + off, si + x1 + off);
+      };
+      x[0] = tap(0);
+#pragma unroll
+      for (int h = 0; h < TCO; h++) a[h] = ld_tr(po + h * 16, po + 16 * LDO + h * 16);
+      x[1] = tap(1);
+#pragma unroll
+      for (int t = 0; t < 9; t++) {  // two taps ahead, and no further: registers
+        if (t + 2 < 9) x[(t + 2) % 3] = tap(t + 2);
+#pragma unroll
+        for (int h = 0; h < TCO; h++)
+          acc[t][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h], x[t % 3], acc[t][h], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (bias)
+#pragma unroll
+        for (int h = 0; h < TCO; h++)
+          accb[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h], ones, accb[h], 0, 0, 0);
+    }
+    __syncthreads();
+  }
+  // wave wk = 1 hands its sums to wave wk = 0, one tap (the bias last) at a time
+  if (WK == 2) {
+    f32x4* const red = reinterpret_cast<f32x4*>(sx) + (size_t)wci * TCO * 64 + lane;
+#pragma unroll
+    for (int t = 0; t < 10; t++) {
+#pragma unroll
+      for (int h = 0; h < TCO; h++)
+        if (wk == 1) red[h * 64] = t < 9 ? acc[t < 9 ? t : 0][h] : accb[h];
+      __syncthreads();
+#pragma unroll
+      for (int h = 0; h < TCO; h++)
+        if (wk == 0) {
+          if (t < 9) acc[t < 9 ? t : 0][h] += red[h * 64];
+          else accb[h] += red[h * 64];
+        }
+      __syncthreads();
+    }
+    if (wk == 1) return;
+  }
+  const size_t n = (size_t)Cout * 9 * Cin + Cout;
+  float* const out = part + (size_t)chunk * n;
+  const unsigned ow = (unsigned)(cob + kb * 4) * 9u * (unsigned)Cin + (unsigned)(cib + wci * 16 + r);
+#pragma unroll
+  for (int h = 0; h < TCO; h++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+#pragma unroll
+      for (int t = 0; t < 9; t++)
+        out[ow + (unsigned)((h * 16 + i) * 9 + t) * (unsigned)Cin] = acc[t][h][i];
+      if (bias && r == 0) out[n - Cout + (cob + h * 16 + kb * 4 + i)] = accb[h][i];
+      __builtin_amdgcn_sched_barrier(0);  // no addresses ahead: registers
+    }
+}
+
 // part[chunk][c] = sum over the chunk's pixels of g[p][c] (bias gradient).
 // Threads are (lane, group) pairs: a group is 8 consecutive channels read as
 // one 16-byte load, lane = t / (C/8) over 256 / (C/8) pixel lanes, so a wave
@@ -1171,28 +1347,105 @@ hipError_t conv3x3(const ConvSrc& cs, const u16* w, const float* bias, const u16
   return hipGetLastError();
 }
 
-int wgrad_tile(int Cout, int Cin) { return Cout % 64 == 0 && Cin % 64 == 0 ? 64 : 32; }
+static int wgrad_tile_edge(int Cout, int Cin) { return Cout % 64 == 0 && Cin % 64 == 0 ? 64 : 32; }
 
-int wgrad_groups(const ConvSrc& cs) {
-  return (int)(((long)cs.B * cs.H * cs.W + WG_PX - 1) / WG_PX);
+// The tile of a weight gradient: up to 128 pixels per wave along K, the least
+// clocks of MFMAs and staged bytes (16 per clock) over all tiles; a tile that
+// leaves a CU one workgroup counts half as much again, for what does not
+// overlap.  512 workgroups fill the CUs once: with 256 the kernels took 16-50 %
+// longer and the sums of the chunks 4 us less each.  False where none fits the
+// LDS (dilations of about 12 and more): k_wgrad and k_wgrad64.
+static bool wgrad_tile_plan(const Src& s, int Cout, WgTile& best, int& best_lds, WgradPlan& p) {
+  constexpr int LDS_MAX = 160 << 10, WGS = 512;
+  const int Cin = s.C0 + s.C1;
+  const int co = Cout % 64 ? 32 : 64, ci = Cin % 64 ? 32 : 64, wk = ci == 64 ? 1 : 2;
+  long best_cost = 0;
+  bool found = false;
+  for (int w = 4; w <= 64; w++) {
+    WgTile t{};
+    t.nx = (s.W + w - 1) / w;
+    t.tw = (s.W + t.nx - 1) / t.nx;
+    if (t.tw < 2) continue;  // inv_tw holds divisors of at least 2
+    t.th = std::min(s.H, 128 * wk / t.tw);
+    t.ny = (s.H + t.th - 1) / t.th;
+    t.th = (s.H + t.ny - 1) / t.ny;
+    t.groups = (t.tw * t.th + 32 * wk - 1) / (32 * wk) * wk;
+    const int row = t.tw + 2 * s.dil;
+    const long npx = (long)row * (t.th + 2 * s.dil);
+    const long lds = (t.groups * 32L * (co + 8) + npx * (ci + 8)) * 2;
+    if (lds > LDS_MAX) continue;
+    const long tiles = (long)s.B * t.nx * t.ny;
+    const long cost = tiles * (t.groups / wk * (co / 16) * 9 * 16L + lds / 16) *
+                      (2 * lds > LDS_MAX ? 3 : 2);
+    if (found && cost >= best_cost) continue;
+    found = true;
+    best_cost = cost;
+    t.tiles = (int)tiles;
+    t.inv_row = inv32(row);
+    t.inv_tw = inv32(t.tw);
+    best = t;
+    best_lds = (int)std::max(lds, (long)co / 16 * (ci / 16) * 1024);  // the sums of the wk waves
+  }
+  if (!found) return false;
+  const long blocks = (long)(Cout / co) * (Cin / ci);
+  const long chunks = std::max(1L, std::min((long)best.tiles, WGS / blocks));
+  best.per_chunk = (int)((best.tiles + chunks - 1) / chunks);
+  p.chunks = (best.tiles + best.per_chunk - 1) / best.per_chunk;
+  p.with_bias = true;
+  return true;
 }
 
-int wgrad_chunks(const ConvSrc& cs, int grp_per_chunk) {
-  return (wgrad_groups(cs) + grp_per_chunk - 1) / grp_per_chunk;
+static int wgrad_groups(const Src& s) {
+  return (int)(((long)s.B * s.H * s.W + WG_PX - 1) / WG_PX);
 }
 
-hipError_t wgrad(const ConvSrc& cs, const u16* dout, int Cout, float* part, int grp_per_chunk,
-                 hipStream_t st) {
-  const int Cin = cs.C0 + cs.C1;
-  if (Cout % 32 || Cin % 32 || grp_per_chunk < 1 ||
-      (long)cs.B * cs.H * cs.W + WG_PX > 0x7fffffffL)
+// Chunks of k_wgrad and k_wgrad64: about 2048 workgroups per launch (fewer
+// chunks = less partial-sum traffic for the fixed-order reduction).
+static int wgrad_grp_per_chunk(const Src& s, int Cout) {
+  const int Cin = s.C0 + s.C1, T = wgrad_tile_edge(Cout, Cin);
+  const long chunks = std::max(1L, 2048 / ((long)(Cout / T) * 9 * (Cin / T)));
+  return (int)std::max(1L, (wgrad_groups(s) + chunks - 1) / chunks);
+}
+
+WgradPlan wgrad_plan(const ConvSrc& cs, int Cout) {
+  const Src s = src_of(cs);
+  WgTile t;
+  int lds;
+  WgradPlan p;
+  if (wgrad_tile_plan(s, Cout, t, lds, p)) return p;
+  const int g = wgrad_grp_per_chunk(s, Cout);
+  p.chunks = (wgrad_groups(s) + g - 1) / g;
+  p.with_bias = false;
+  return p;
+}
+
+hipError_t wgrad(const ConvSrc& cs, const u16* dout, int Cout, float* part, hipStream_t st) {
+  const Src s = src_of(cs);
+  const int Cin = s.C0 + s.C1;
+  if (Cout % 32 || Cin % 32 || (long)cs.B * cs.H * cs.W + WG_PX > 0x7fffffffL)
     return hipErrorInvalidValue;
-  const int T = wgrad_tile(Cout, Cin);
-  const long nwork = (long)wgrad_chunks(cs, grp_per_chunk) * (Cout / T) * 9 * (Cin / T);
+  WgTile t;
+  int lds;
+  WgradPlan p;
+  if (wgrad_tile_plan(s, Cout, t, lds, p)) {
+    const int nwork = p.chunks * (Cout / (Cout % 64 ? 32 : 64)) * (Cin / (Cin % 64 ? 32 : 64));
+    const unsigned g = (unsigned)((nwork + 7) / 8 * 8);  // a multiple of 8, dealt to the XCDs
+    if (Cout % 64 == 0 && Cin % 64 == 0)
+      k_wgrad_tile<4, 4, 1><<<g, 256, lds, st>>>(s, cb(dout), Cout, part, t, nwork);
+    else if (Cout % 64 == 0)
+      k_wgrad_tile<4, 2, 2><<<g, 256, lds, st>>>(s, cb(dout), Cout, part, t, nwork);
+    else if (Cin % 64 == 0)
+      k_wgrad_tile<2, 4, 1><<<g, 256, lds, st>>>(s, cb(dout), Cout, part, t, nwork);
+    else
+      k_wgrad_tile<2, 2, 2><<<g, 256, lds, st>>>(s, cb(dout), Cout, part, t, nwork);
+    return hipGetLastError();
+  }
+  const int T = wgrad_tile_edge(Cout, Cin), per = wgrad_grp_per_chunk(s, Cout);
+  const long nwork = (long)((wgrad_groups(s) + per - 1) / per) * (Cout / T) * 9 * (Cin / T);
   if (nwork > 0x7ffffff0L) return hipErrorInvalidValue;
   const unsigned g = (unsigned)((nwork + 7) / 8 * 8);  // a multiple of 8 (wgrad_item)
-  if (T == 64) k_wgrad64<<<g, 256, 0, st>>>(src_of(cs), cb(dout), Cout, part, grp_per_chunk, (int)nwork);
-  else k_wgrad<<<g, 256, 0, st>>>(src_of(cs), cb(dout), Cout, part, grp_per_chunk, (int)nwork);
+  if (T == 64) k_wgrad64<<<g, 256, 0, st>>>(s, cb(dout), Cout, part, per, (int)nwork);
+  else k_wgrad<<<g, 256, 0, st>>>(s, cb(dout), Cout, part, per, (int)nwork);
   return hipGetLastError();
 }
 

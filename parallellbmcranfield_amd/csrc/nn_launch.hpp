@@ -25,14 +25,15 @@ struct ConvSrc {
 // be null.
 hipError_t conv3x3(const ConvSrc& s, const u16* w, const float* bias, const u16* mask, u16* out,
                    int Cout, bool relu, hipStream_t st);
-// Weight-gradient partial sums, one [Cout][9][Cin] block per chunk of
-// grp_per_chunk groups of 64 consecutive pixels (Cout, Cin multiples of 32).
-// (co, ci) tile edge of a workgroup: 64 when both counts are multiples of 64
-int wgrad_tile(int Cout, int Cin);
-int wgrad_groups(const ConvSrc& s);
-int wgrad_chunks(const ConvSrc& s, int grp_per_chunk);
-hipError_t wgrad(const ConvSrc& s, const u16* dout, int Cout, float* part, int grp_per_chunk,
-                 hipStream_t st);
+// Weight-gradient partial sums into part, [chunks][Cout][9][Cin]; with_bias:
+// each chunk's block is followed by its Cout sums of the bias gradient
+// (Cout, Cin multiples of 32).
+struct WgradPlan {
+  int chunks = 0;
+  bool with_bias = false;
+};
+WgradPlan wgrad_plan(const ConvSrc& s, int Cout);
+hipError_t wgrad(const ConvSrc& s, const u16* dout, int Cout, float* part, hipStream_t st);
 hipError_t colsum_part(const u16* g, int P, int C, int px_per_chunk, float* part, hipStream_t st);
 hipError_t reduce_chunks(const float* part, int nchunk, long n, float* out, hipStream_t st);
 // wf: the BF16 weights of a conv, packed for conv3x3; wt: its data gradient's.
