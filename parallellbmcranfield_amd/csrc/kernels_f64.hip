@@ -92,24 +92,46 @@ __global__ void k_ref_residual(const double* __restrict__ cres, int m, int n,
 // Velocity-change sums of each batched instance over its storage rectangle:
 // out[2k] = sum |u(t) - u(t-K)|^2, out[2k+1] = sum |u(t)|^2, from the per-cell
 // terms the residual step leaves in planes 3 and 4 of the snapshot.  One
-// workgroup per instance, fixed order: the sums are deterministic.
-__global__ __launch_bounds__(256) void k_inst_resid(const double* __restrict__ snap, int plane,
-                                                    int pitch, const int* __restrict__ rect,
-                                                    const uint8_t* __restrict__ active,
-                                                    double* __restrict__ out) {
+// workgroup per instance, fixed order: the sums are deterministic.  Bound by
+// the latency of its loads: 1024 threads, eight loads in flight each, cells
+// stepped through without a division (48 instances of 25 600 cells: 90 us
+// with 256 threads and a 64-bit division per cell, now 16).
+constexpr int IR_NT = 1024, IR_U = 4;
+__global__ __launch_bounds__(IR_NT) void k_inst_resid(const double* __restrict__ snap, int plane,
+                                                      int pitch, const int* __restrict__ rect,
+                                                      const uint8_t* __restrict__ active,
+                                                      double* __restrict__ out) {
   const int k = blockIdx.x;
   const int x0 = rect[4 * k], y0 = rect[4 * k + 1], w = rect[4 * k + 2], h = rect[4 * k + 3];
   double a = 0.0, b = 0.0;
   if (active[k]) {
-    const long cnt = (long)w * h;
-    for (long e = threadIdx.x; e < cnt; e += 256) {
-      const long r = e / w, c = e - r * w;
-      const long idx = (y0 + r) * (long)pitch + x0 + c;
-      a += snap[3 * (size_t)plane + idx];
-      b += snap[4 * (size_t)plane + idx];
+    const double* da = snap + 3 * (size_t)plane + (size_t)y0 * pitch + x0;
+    const double* db = da + plane;
+    const int dr = IR_NT / w, dc = IR_NT - dr * w;  // IR_NT cells on
+    int r = (int)threadIdx.x / w, c = (int)threadIdx.x - r * w;
+    while (r < h) {
+      double va[IR_U], vb[IR_U];
+#pragma unroll
+      for (int u = 0; u < IR_U; u++) {
+        const bool in = r < h;
+        const size_t at = in ? (size_t)r * pitch + c : 0;
+        va[u] = in ? da[at] : 0.0;
+        vb[u] = in ? db[at] : 0.0;
+        r += dr;
+        c += dc;
+        if (c >= w) {
+          c -= w;
+          r++;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < IR_U; u++) {
+        a += va[u];
+        b += vb[u];
+      }
     }
   }
-  __shared__ double red[4][2];
+  __shared__ double red[IR_NT / 64][2];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   a = wave_sum(a);
   b = wave_sum(b);
@@ -120,7 +142,7 @@ __global__ __launch_bounds__(256) void k_inst_resid(const double* __restrict__ s
   __syncthreads();
   if (threadIdx.x < 2) {
     double s = 0.0;
-    for (int w2 = 0; w2 < 4; w2++) s += red[w2][threadIdx.x];
+    for (int w2 = 0; w2 < IR_NT / 64; w2++) s += red[w2][threadIdx.x];
     out[2 * k + threadIdx.x] = s;
   }
 }
@@ -128,7 +150,7 @@ __global__ __launch_bounds__(256) void k_inst_resid(const double* __restrict__ s
 hipError_t launch_inst_resid(const double* snap, int plane, int pitch, const int* rect,
                              const uint8_t* active, int ninst, double* out, hipStream_t st) {
   if (ninst <= 0) return hipSuccess;
-  k_inst_resid<<<ninst, 256, 0, st>>>(snap, plane, pitch, rect, active, out);
+  k_inst_resid<<<ninst, IR_NT, 0, st>>>(snap, plane, pitch, rect, active, out);
   return hipGetLastError();
 }
 

@@ -35,7 +35,7 @@ static int launch_step_passes(lbm_solver* s, const Launch& L);
 
 namespace {
 
-constexpr int HCAP = 1024;  // device history slots
+constexpr int HCAP = 1024;  // history slots
 constexpr int HW = 8;       // slot: raw residual [0..3], force [4..5], unused [6..7]
 
 int dev_alloc(lbm_solver* s, void** p, size_t bytes) {
@@ -140,12 +140,9 @@ bool finalize_resid(lbm_solver* s, const double raw[4], double r[4]) {
 
 int flush_history(lbm_solver* s) {
   if (s->pending == 0) return LBM_OK;
-  std::vector<double> raw((size_t)s->pending * HW);
-  HC(hipMemcpyAsync(raw.data(), s->d_hist, raw.size() * sizeof(double), hipMemcpyDeviceToHost,
-                    s->stream));
   HC(hipStreamSynchronize(s->stream));
   for (int i = 0; i < s->pending; i++) {
-    const double* row = &raw[(size_t)i * HW];
+    const double* row = s->hist + (size_t)i * HW;
     const int what = s->pending_what[i];
     if ((what & 2) && !s->diverged) {
       s->force_iter.push_back(s->pending_iter[i]);
@@ -1067,7 +1064,13 @@ static int solver_create(const lbm_case* c, const lbm_options* o, const double* 
   if (!rc) rc = dev_alloc(s, (void**)&s->d_u, sizeof(double) * (size_t)s->plane);
   if (!rc) rc = dev_alloc(s, (void**)&s->d_v, sizeof(double) * (size_t)s->plane);
   if (!rc) rc = dev_alloc(s, (void**)&s->d_part, sizeof(double) * 6 * (size_t)s->nparts);
-  if (!rc) rc = dev_alloc(s, (void**)&s->d_hist, sizeof(double) * HW * HCAP);
+  // the kernels write their sums where the host reads them: no copy behind an
+  // evaluation, only the wait
+  if (!rc)
+    rc = check_hip(hipHostMalloc((void**)&s->hist, sizeof(double) * (HW * HCAP + 2 * (size_t)ninst),
+                                 hipHostMallocDefault),
+                   "residual rows");
+  if (!rc) s->inst_raw = s->hist + HW * HCAP;
   if (!rc && s->prec == LBM_PREC_F16_SR) {  // step number of stochastic rounding, 2 slots
     rc = dev_alloc(s, (void**)&s->d_seed, 2 * sizeof(uint32_t));
     if (!rc) rc = check_hip(hipMemset(s->d_seed, 0, 2 * sizeof(uint32_t)), "clear step number");
@@ -1085,7 +1088,6 @@ static int solver_create(const lbm_case* c, const lbm_options* o, const double* 
     if (!rc) rc = dev_alloc(s, (void**)&s->d_tile_inst, sizeof(uint16_t) * tile_inst.size());
     if (!rc) rc = dev_alloc(s, (void**)&s->d_inst_active, (size_t)ninst);
     if (!rc) rc = dev_alloc(s, (void**)&s->d_inst_rect, sizeof(int) * srect.size());
-    if (!rc) rc = dev_alloc(s, (void**)&s->d_inst_res, sizeof(double) * 4 * (size_t)ninst);
     if (!rc) rc = dev_alloc(s, (void**)&s->d_tile_list, sizeof(uint32_t) * ((size_t)s->nb_bulk + align));
     if (!rc) rc = check_hip(hipMemcpy(s->d_inst_par, inst_par.data(), sizeof(float) * inst_par.size(), hipMemcpyHostToDevice), "upload");
     if (!rc) rc = check_hip(hipMemcpy(s->d_node_inst, node_inst.data(), sizeof(uint16_t) * node_inst.size(), hipMemcpyHostToDevice), "upload");
@@ -1514,8 +1516,8 @@ void lbm_solver_destroy(lbm_solver* s) {
   if (s->stream) (void)hipStreamSynchronize(s->stream);
   void* ptrs[] = {s->buf[0], s->buf[1], s->d_cls, s->d_tflag, s->d_bn, s->d_on, s->d_orow, s->d_side,
                   s->d_rho, s->d_u, s->d_v, s->d_f, s->d_metaf, s->d_snap, s->d_cres,
-                  s->d_part, s->d_hist, s->d_inst_par, s->d_tile_inst, s->d_node_inst,
-                  s->d_inst_active, s->d_inst_rect, s->d_inst_res, s->d_tile_list,
+                  s->d_part, s->d_inst_par, s->d_tile_inst, s->d_node_inst,
+                  s->d_inst_active, s->d_inst_rect, s->d_tile_list,
                   s->d_wmask, s->d_seed, s->d_tiles, s->d_cls_two, s->buf3, s->d_cls_b[0], s->d_cls_b[1],
                   s->d_tflag_b[0], s->d_tflag_b[1], s->d_list_b[0], s->d_list_b[1],
                   s->d_tiles3, s->d_cls_three, s->buf4, s->d_cls_b3[0], s->d_cls_b3[1],
@@ -1523,6 +1525,7 @@ void lbm_solver_destroy(lbm_solver* s) {
                   s->d_list_b3[0], s->d_list_b3[1], s->d_list_b3[2], s->d_rule, s->d_body};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
+  if (s->hist) (void)hipHostFree(s->hist);
   for (hipEvent_t e : s->ev) (void)hipEventDestroy(e);
   for (hipGraphExec_t g : s->gexec)
     if (g) (void)hipGraphExecDestroy(g);
@@ -1577,10 +1580,7 @@ static int rebuild_tile_list(lbm_solver* s) {
 static int batch_eval(lbm_solver* s) {
   const int ni = s->ninst;
   HC(launch_inst_resid(s->d_snap, s->plane, s->pitch, s->d_inst_rect, s->d_inst_active, ni,
-                       s->d_inst_res, s->stream));
-  std::vector<double> raw(2 * (size_t)ni);
-  HC(hipMemcpyAsync(raw.data(), s->d_inst_res, raw.size() * sizeof(double), hipMemcpyDeviceToHost,
-                    s->stream));
+                       s->inst_raw, s->stream));
   HC(hipStreamSynchronize(s->stream));
   const double now = wall_seconds() - s->t_first_step;
   const double K = (double)s->opt.resid_every;
@@ -1590,7 +1590,7 @@ static int batch_eval(lbm_solver* s) {
   std::vector<int> rect(4 * (size_t)ni);
   for (int k = 0; k < ni; k++) {
     if (!s->inst_active[k]) continue;
-    const double a = raw[2 * k], b = raw[2 * k + 1];
+    const double a = s->inst_raw[2 * k], b = s->inst_raw[2 * k + 1];
     const double r = b > 0 ? std::sqrt(a) / (K * std::sqrt(b)) : std::sqrt(a);
     s->inst_res[k] = r;
     if (!(r == r)) {  // this instance diverged: stop it, the others go on
@@ -1683,7 +1683,7 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
       Launch L = make_launch(s, s->cur);
       L.body = s->d_body;
       L.nbody = s->nbody;
-      L.hist = s->d_hist + (size_t)s->pending * HW;
+      L.hist = s->hist + (size_t)s->pending * HW;
       HC(s->prec == 0 ? launch_pass_f64(1, MODE_RESID, PASS_FORCE, L)
                       : launch_pass_lp(s->prec, 1, MODE_RESID, PASS_FORCE, L));
       s->pending_iter.push_back(s->iter);
@@ -1837,7 +1837,7 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
     HC(pass(s, mode, PASS_OUTLET, L));
     const bool row_r = reval && !s->ninst;  // batched residuals are per instance
     if (row_r || feval) {
-      double* slot = s->d_hist + (size_t)s->pending * HW;
+      double* slot = s->hist + (size_t)s->pending * HW;
       if (mode == MODE_RESID) HC(launch_reduce_partials(s->d_part, s->nparts, slot, s->stream));
       if (row_r && rk == LBM_RESID_REFERENCE)
         HC(launch_ref_residual(s->d_cres, s->cs->m, s->cs->n, slot, s->stream));
