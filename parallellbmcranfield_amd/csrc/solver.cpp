@@ -218,7 +218,13 @@ int observe(lbm_solver* s, bool with_f) {
     L.out.f = s->d_f;
     L.out.metaf = s->d_metaf;
   }
-  for (int p = 0; p < 3; p++) HC(pass(s, MODE_OBSERVE, p, L));
+  if (s->fused) {  // as a step: list nodes and bulk tiles in one launch
+    HC(pass(s, MODE_OBSERVE, PASS_FUSED, L));
+  } else {
+    HC(pass(s, MODE_OBSERVE, PASS_BULK, L));
+    HC(pass(s, MODE_OBSERVE, PASS_BOUNDARY, L));
+  }
+  HC(pass(s, MODE_OBSERVE, PASS_OUTLET, L));
   s->observed = s->iter;
   if (with_f) s->observed_f = s->iter;
   return LBM_OK;
@@ -1060,9 +1066,11 @@ static int solver_create(const lbm_case* c, const lbm_options* o, const double* 
   if (!rc) rc = dev_alloc(s, (void**)&s->d_on, sizeof(BNode) * std::max(1, s->non));
   if (!rc) rc = dev_alloc(s, (void**)&s->d_orow, sizeof(int) * orow.size());
   if (!rc) rc = dev_alloc(s, &s->d_side, rsz * 9 * (size_t)nside);
-  if (!rc) rc = dev_alloc(s, (void**)&s->d_rho, sizeof(double) * (size_t)s->plane);
-  if (!rc) rc = dev_alloc(s, (void**)&s->d_u, sizeof(double) * (size_t)s->plane);
-  if (!rc) rc = dev_alloc(s, (void**)&s->d_v, sizeof(double) * (size_t)s->plane);
+  if (!rc) rc = dev_alloc(s, (void**)&s->d_rho, sizeof(double) * 3 * (size_t)s->plane);
+  if (!rc) {
+    s->d_u = s->d_rho + s->plane;
+    s->d_v = s->d_u + s->plane;
+  }
   if (!rc) rc = dev_alloc(s, (void**)&s->d_part, sizeof(double) * 6 * (size_t)s->nparts);
   // the kernels write their sums where the host reads them: no copy behind an
   // evaluation, only the wait
@@ -1152,8 +1160,9 @@ static int solver_create(const lbm_case* c, const lbm_options* o, const double* 
     }
   }
   {
-    std::vector<double> pr((size_t)s->plane, 0.0), pu((size_t)s->plane, 0.0),
-        pv((size_t)s->plane, 0.0);
+    std::vector<double> pr(3 * (size_t)s->plane, 0.0);
+    double* const pu = pr.data() + s->plane;
+    double* const pv = pu + s->plane;
     for (int j = 0; j < m; j++)
       for (int i = 0; i < n; i++) {
         const size_t idx = (size_t)(j + 1) * s->pitch + (i + 1);
@@ -1162,14 +1171,9 @@ static int solver_create(const lbm_case* c, const lbm_options* o, const double* 
         pu[idx] = s->u0[lin];
         pv[idx] = s->v0[lin];
       }
-    rc = check_hip(hipMemcpy(s->d_rho, pr.data(), sizeof(double) * s->plane, hipMemcpyHostToDevice), "upload rho");
-    if (!rc) rc = check_hip(hipMemcpy(s->d_u, pu.data(), sizeof(double) * s->plane, hipMemcpyHostToDevice), "upload u");
-    if (!rc) rc = check_hip(hipMemcpy(s->d_v, pv.data(), sizeof(double) * s->plane, hipMemcpyHostToDevice), "upload v");
-    if (!rc && s->d_snap) {
-      rc = check_hip(hipMemcpy(s->d_snap, pr.data(), sizeof(double) * s->plane, hipMemcpyHostToDevice), "snap");
-      if (!rc) rc = check_hip(hipMemcpy(s->d_snap + s->plane, pu.data(), sizeof(double) * s->plane, hipMemcpyHostToDevice), "snap");
-      if (!rc) rc = check_hip(hipMemcpy(s->d_snap + 2 * (size_t)s->plane, pv.data(), sizeof(double) * s->plane, hipMemcpyHostToDevice), "snap");
-    }
+    rc = check_hip(hipMemcpy(s->d_rho, pr.data(), sizeof(double) * pr.size(), hipMemcpyHostToDevice), "upload rho, u, v");
+    if (!rc && s->d_snap)
+      rc = check_hip(hipMemcpy(s->d_snap, pr.data(), sizeof(double) * pr.size(), hipMemcpyHostToDevice), "snap");
   }
   if (!rc) rc = check_hip(hipMemcpy(s->d_cls, cls.data(), cls.size(), hipMemcpyHostToDevice), "upload classes");
   if (!rc) rc = check_hip(hipMemcpy(s->d_tflag, tflag.data(), tflag.size(), hipMemcpyHostToDevice), "upload tile flags");
@@ -1515,7 +1519,7 @@ void lbm_solver_destroy(lbm_solver* s) {
   if (!s) return;
   if (s->stream) (void)hipStreamSynchronize(s->stream);
   void* ptrs[] = {s->buf[0], s->buf[1], s->d_cls, s->d_tflag, s->d_bn, s->d_on, s->d_orow, s->d_side,
-                  s->d_rho, s->d_u, s->d_v, s->d_f, s->d_metaf, s->d_snap, s->d_cres,
+                  s->d_rho, s->d_f, s->d_metaf, s->d_snap, s->d_cres,
                   s->d_part, s->d_inst_par, s->d_tile_inst, s->d_node_inst,
                   s->d_inst_active, s->d_inst_rect, s->d_tile_list,
                   s->d_wmask, s->d_seed, s->d_tiles, s->d_cls_two, s->buf3, s->d_cls_b[0], s->d_cls_b[1],
