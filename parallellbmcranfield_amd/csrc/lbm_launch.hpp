@@ -58,10 +58,12 @@ enum Pass {
 enum Mode { MODE_STEP = 0, MODE_RESID = 1, MODE_OBSERVE = 2 };
 
 // Region shapes of the LDS-resident steps (RX x RY nodes per workgroup).
+// Blocks of interior nodes may have wider regions (plain_rx), which keep their
+// state in registers.
 struct LdsShape {
-  int rx, ry;
+  int rx, ry, plain_rx;
 };
-constexpr LdsShape LDS_SHAPES[] = {{32, 16}, {32, 32}, {64, 32}};
+constexpr LdsShape LDS_SHAPES[] = {{32, 16, 32}, {32, 32, 32}, {64, 32, 64}, {32, 32, 64}};
 
 // prec: 0 F64, 1 F32, 2 F16.  coll: 1 BGKW, 2 TRT, 3 MRT.
 hipError_t launch_pass(int prec, int coll, int mode, int pass, const Launch& L);

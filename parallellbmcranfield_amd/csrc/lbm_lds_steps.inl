@@ -54,6 +54,23 @@ __device__ inline void lds_node(typename S::R (&F)[9], uint32_t r, const LdsList
     node_dev<COLL>(F, p.rho0_f, 1.f, 1.f, still, list, cp, out);
 }
 
+// The value of the lane DX to the left (DX = 1) or right (-1) in the wave; the
+// wave's outermost lanes keep their own.
+template <int DX, class R>
+__device__ inline R lane_pull(R x) {
+  if constexpr (DX == 0) return x;
+  constexpr int CTRL = DX > 0 ? 0x138 : 0x130;  // wave_shr:1, wave_shl:1
+  constexpr int WORDS = sizeof(R) / 4;
+  struct Words {
+    int w[WORDS];
+  };
+  Words a = __builtin_bit_cast(Words, x);
+#pragma unroll
+  for (int i = 0; i < WORDS; i++)
+    a.w[i] = __builtin_amdgcn_update_dpp(a.w[i], a.w[i], CTRL, 0xf, 0xf, false);
+  return __builtin_bit_cast(R, a);
+}
+
 // steps (1 .. halo + 1) plain steps of one block.  The workgroup works on a
 // region of RX x RY nodes: the block's output nodes and `halo` nodes around
 // them.  Step 1 pulls from METAF_t in memory and leaves its results in LDS;
@@ -74,6 +91,15 @@ __device__ inline void lds_node(typename S::R (&F)[9], uint32_t r, const LdsList
 // three steps and two-step launches as much per two: 4097^2 FP32 MRT 115.2 ->
 // 63.2 us per step (145 -> 265 GLUPS), 2049^2 39.7 -> 19.2, 1025^2 15.2 -> 7.0;
 // FP64 BGK 4097^2 274 -> 145, 2049^2 72 -> 39; FP16 BGK 4097^2 111.8 -> 56.4.
+// LANES (FP64): 72 bytes of LDS per node and step's 18 accesses limited FP64
+// to regions of 32 x 32, which form 1.69 nodes per node kept and read 1.78.
+// Blocks of interior nodes now hold their state in registers, a wave 64 x 4
+// nodes, and a third of the LDS accesses is left for two nodes per thread, a
+// sixth for four: FP64 BGK 4097^2 146.5 -> 130.6 us per step, 2049^2 40.2 ->
+// 37.0, 1025^2 11.2 -> 9.9; there memory and VALU issue bound it together
+// (34 bytes per node and step: 4.4 TB/s).  FP32 and FP16 keep the LDS form: the
+// DPP moves are VALU instructions, which bound them (FP32 MRT 4097^2 63.2
+// against 68.8 us).
 // Ordinary stores: two blocks store parts of a cache line where they meet,
 // and non-temporal stores gave those to memory one by one (4097^2 FP32 82.7
 // against 63.2 us per step, FP64 165.6 against 144.8).
@@ -81,7 +107,7 @@ __device__ inline void lds_node(typename S::R (&F)[9], uint32_t r, const LdsList
 // with one, 1025^2 FP32 took 8.3 us per step against 6.7.  One LDS copy and two
 // barriers per step; two copies and one barrier measured 0-25 % slower (half
 // the workgroups per CU).
-template <class S, int COLL, int NT, int RX, int NPT, bool GEN>
+template <class S, int COLL, int NT, int RX, int NPT, bool GEN, bool LANES>
 __device__ inline void lds_block(const typename S::T* __restrict__ src,
                                  typename S::T* __restrict__ dst,
                                  const uint32_t* __restrict__ rule, const LdsTile& tl,
@@ -167,42 +193,86 @@ __device__ inline void lds_block(const typename S::T* __restrict__ src,
       for (int k = 0; k < 9; k++) v[i][k] = out[k];
     }
   }
-  R* const w = lds + RX + 1 + ly * RX + lx;
-  for (int t = 1; t < steps; t++) {
-    // step t's results to LDS (a cell without a node keeps the solid value
-    // it was loaded with)
-    if (wfar <= steps - t) {
+  if constexpr (LANES) {
+    // What a node pulls from its own thread's or its wave's nodes stays in
+    // registers, across lanes by DPP moves: the lanes that get a wrong
+    // neighbour are the region's outermost columns, which no step from the
+    // second on has to form.  LDS carries what crosses the threads' upper and
+    // lower edges, in two copies in turn, so that one barrier per step is
+    // enough.
+    static_assert(!GEN && RX <= 64);
+    constexpr int NG = NT / RX, QL = (NG + 2) * RX;
+    constexpr int SLOT[9] = {0, 0, 0, 0, 3, 1, 2, 4, 5};
+    for (int t = 1; t < steps; t++) {
+      R* const w = lds + 1 + (t & 1) * 6 * QL + ((int)threadIdx.x / RX + 1) * RX + lx;
+      if (wfar <= steps - t) {
 #pragma unroll
-      for (int i = 0; i < NPT; i++) {
-        const bool node = !GEN || (rl[i] & LR_CLASS) != 0u;
-        if (GEN && (far[i] > steps - t || (t > 1 && !node))) continue;
-        if (node) S::round_raw(v[i], idx[i], step0 + (uint32_t)(t - 1));
+        for (int i = 0; i < NPT; i++) S::round_raw(v[i], idx[i], step0 + (uint32_t)(t - 1));
 #pragma unroll
-        for (int k = 0; k < 9; k++) w[k * PL + i * RX] = v[i][k];
+        for (int k = 0; k < 9; k++)
+          if (CY[k] != 0) w[SLOT[k] * QL] = v[CY[k] > 0 ? NPT - 1 : 0][k];
       }
-    }
-    __syncthreads();
-    if (wfar < steps - t) {
+      __syncthreads();
+      if (wfar < steps - t) {
+        R below[9];  // the values before this step of the node below
 #pragma unroll
-      for (int i = 0; i < NPT; i++) {
-        if (!forms(i, steps - t - 1)) continue;
-        const R* wi = w + i * RX;
-        R F[9];
+        for (int i = 0; i < NPT; i++) {
+          R F[9];
 #pragma unroll
-        for (int k = 0; k < 9; k++) F[k] = wi[k * PL - CX[k] - CY[k] * RX];
-        if (GEN && (rl[i] & LR_CLASS) != LR_INTERIOR) {
-#pragma unroll
-          for (int k = 0; k < 9; k++)
-            if (!((rl[i] >> k) & 1)) F[k] = wi[k * PL];
+          for (int k = 0; k < 9; k++) {
+            if (CY[k] > 0 && i == 0)
+              F[k] = w[SLOT[k] * QL - CX[k] - RX];
+            else if (CY[k] < 0 && i == NPT - 1)
+              F[k] = w[SLOT[k] * QL - CX[k] + RX];
+            else {
+              const R x = CY[k] > 0 ? below[k] : (CY[k] < 0 ? v[i + 1 < NPT ? i + 1 : i][k] : v[i][k]);
+              F[k] = CX[k] == 0 ? x : (CX[k] > 0 ? lane_pull<1>(x) : lane_pull<-1>(x));
+            }
+            below[k] = v[i][k];
+          }
+          lds_node<S, COLL, false>(
+              F, rl[i], ll, bn, p, cp, [&](int) { return R(0); }, [&](int) { return R(0); }, v[i]);
         }
-        if constexpr (GEN && NPT > 1)
-          if ((rl[i] & LR_CLASS) == LR_LIST) ll = list[rl[i] >> LR_SHIFT];
-        lds_node<S, COLL, GEN>(
-            F, rl[i], ll, bn, p, cp, [&](int k) { return wi[k * PL]; },
-            [&](int k) { return wi[k * PL - CX[k] - CY[k] * RX]; }, v[i]);
       }
     }
-    __syncthreads();
+  } else {
+    R* const w = lds + RX + 1 + ly * RX + lx;
+    for (int t = 1; t < steps; t++) {
+      // step t's results to LDS (a cell without a node keeps the solid value
+      // it was loaded with)
+      if (wfar <= steps - t) {
+#pragma unroll
+        for (int i = 0; i < NPT; i++) {
+          const bool node = !GEN || (rl[i] & LR_CLASS) != 0u;
+          if (GEN && (far[i] > steps - t || (t > 1 && !node))) continue;
+          if (node) S::round_raw(v[i], idx[i], step0 + (uint32_t)(t - 1));
+#pragma unroll
+          for (int k = 0; k < 9; k++) w[k * PL + i * RX] = v[i][k];
+        }
+      }
+      __syncthreads();
+      if (wfar < steps - t) {
+#pragma unroll
+        for (int i = 0; i < NPT; i++) {
+          if (!forms(i, steps - t - 1)) continue;
+          const R* wi = w + i * RX;
+          R F[9];
+#pragma unroll
+          for (int k = 0; k < 9; k++) F[k] = wi[k * PL - CX[k] - CY[k] * RX];
+          if (GEN && (rl[i] & LR_CLASS) != LR_INTERIOR) {
+#pragma unroll
+            for (int k = 0; k < 9; k++)
+              if (!((rl[i] >> k) & 1)) F[k] = wi[k * PL];
+          }
+          if constexpr (GEN && NPT > 1)
+            if ((rl[i] & LR_CLASS) == LR_LIST) ll = list[rl[i] >> LR_SHIFT];
+          lds_node<S, COLL, GEN>(
+              F, rl[i], ll, bn, p, cp, [&](int k) { return wi[k * PL]; },
+              [&](int k) { return wi[k * PL - CX[k] - CY[k] * RX]; }, v[i]);
+        }
+      }
+      __syncthreads();
+    }
   }
 #pragma unroll
   for (int i = 0; i < NPT; i++) {
@@ -211,15 +281,19 @@ __device__ inline void lds_block(const typename S::T* __restrict__ src,
   }
 }
 
-template <class S, int COLL, int NT, int RX, int NPT, int WPE>
+// PRX, PNPT: the regions of blocks of interior nodes, LANES: held in registers
+template <class S, int COLL, int NT, int RX, int NPT, int WPE, int PRX = RX, int PNPT = NPT,
+          bool LANES = false>
 __global__ __launch_bounds__(NT, WPE) void k_lds_steps(
     const typename S::T* __restrict__ src, typename S::T* __restrict__ dst,
     const uint32_t* __restrict__ rule, const LdsTile* __restrict__ tiles,
     const LdsList* __restrict__ list, const BNode* __restrict__ bn, int halo, int steps,
     KParams p) {
   using R = typename S::R;
-  // a row and a cell before and after: pulls of nodes that come to nothing
-  __shared__ R lds[9 * NT * NPT + 2 * (RX + 1)];
+  // a row and a cell before and after (LANES: one row and one cell): pulls of
+  // nodes that come to nothing
+  constexpr int ALL = 9 * NT * NPT + 2 * (RX + 1), EDGES = 12 * (NT + 2 * PRX) + 2;
+  __shared__ R lds[LANES && EDGES > ALL ? EDGES : ALL];
   const uint32_t step0 = step_number<S>(p);
   if constexpr (S::SR) {
     if (blockIdx.x == 0 && threadIdx.x == 0) p.seed[p.seed_slot ^ 1] = step0 + (uint32_t)steps;
@@ -227,10 +301,10 @@ __global__ __launch_bounds__(NT, WPE) void k_lds_steps(
   const LdsTile tl = tiles[blockIdx.x];
   if (tl.x1 <= tl.x0) return;
   if (tl.plain)
-    lds_block<S, COLL, NT, RX, NPT, false>(src, dst, rule, tl, list, bn, halo, steps, p, step0,
+    lds_block<S, COLL, NT, PRX, PNPT, false, LANES>(src, dst, rule, tl, list, bn, halo, steps, p, step0,
                                            lds);
   else
-    lds_block<S, COLL, NT, RX, NPT, true>(src, dst, rule, tl, list, bn, halo, steps, p, step0,
+    lds_block<S, COLL, NT, RX, NPT, true, false>(src, dst, rule, tl, list, bn, halo, steps, p, step0,
                                           lds);
 }
 

@@ -359,8 +359,12 @@ static int rebuild_lds_tiles(lbm_solver* s) {
 // launch as still leave a few rows of output.  From a few hundred thousand
 // cells the chip is full and the nodes formed more than once weigh most:
 // larger regions and fewer steps, fewest where a step moves least (FP16) or
-// a node costs most (stochastic rounding).  FP64 keeps 32 x 32 (64 x 32
-// leaves one workgroup per CU).  Measured, us per step, regions 32 x 16 /
+// a node costs most (stochastic rounding).  FP64 keeps 32 x 32 in LDS (64 x 32
+// leaves one workgroup per CU) and takes 64 x 32 in registers for blocks of
+// interior nodes: BGK 700^2 7.1 -> 6.2 at halo 3 (7.6 at 4), 1025^2 11.2 -> 9.9
+// at halo 4 (10.7 at 3 and 5), 2049^2 40.2 -> 37.0, 4097^2 146.5 -> 130.6; MRT
+// 2049^2 45.2 -> 39.8.  TRT needs more registers than two workgroups leave and
+// stays at 32 x 32 (46.2 -> 44.8).  Measured, us per step, regions 32 x 16 /
 // 32 x 32 / 64 x 32 at their best halo: FP64 BGK 129^2 1.50 / 2.88 / 4.1,
 // 361^2 2.75 / 3.5 / -, 725^2 7.9 / 7.7 / -, 1025^2 13.2 / 12.7 / 14.7; FP32
 // MRT 129^2 1.20 / 1.96 / 2.8, 361^2 1.91 / 2.38 / 2.9, 725^2 4.98 / 4.65 /
@@ -378,6 +382,9 @@ static void pick_lds_shape(lbm_solver* s, long long cells) {
   } else if (cells < (sr ? 1200000 : 400000)) {
     s->lds_shape = 0;
     s->lds_halo = sr ? 2 : 3;
+  } else if (f64 && !s->ninst && s->coll != LBM_TRT) {
+    s->lds_shape = 3;
+    s->lds_halo = cells < 800000 ? 3 : 4;
   } else if (f64 || (s->ninst && !sr)) {
     s->lds_shape = 1;
     s->lds_halo = 4;
@@ -399,7 +406,8 @@ static int setup_lds_steps(lbm_solver* s, const std::vector<uint8_t>& cls,
     return LBM_OK;
   pick_lds_shape(s, (long long)n * m);
   const LdsShape sh = LDS_SHAPES[s->lds_shape];
-  const int h = s->lds_halo, bw = sh.rx - 2 * h, bh = sh.ry - 2 * h;
+  const int h = s->lds_halo, bw = sh.rx - 2 * h, pw = sh.plain_rx - 2 * h;
+  const int bh = sh.ry - 2 * h;
   std::vector<int> rects;
   if (s->ninst)
     for (int k = 0; k < s->ninst; k++) {
@@ -416,28 +424,38 @@ static int setup_lds_steps(lbm_solver* s, const std::vector<uint8_t>& cls,
     for (int y = r[1]; y < r[3] && s->ninst; y++)
       for (int x = r[0]; x < r[2]; x += (y == r[1] || y == r[3] - 1) ? 1 : r[2] - r[0] - 1)
         if (cls[(size_t)y * pitch + x] != 0) return LBM_OK;
+    // the block of output nodes from (x, y), w wide; false where it is left out:
+    // no node, or not `plain` where only such a block is asked for
+    auto add = [&](int x, int y, int w, bool only_plain) {
+      LdsTile t;
+      t.x0 = x;
+      t.y0 = y;
+      t.x1 = std::min(x + w, r[2] - 1);
+      t.y1 = std::min(y + bh, r[3] - 1);
+      t.rx0 = r[0];
+      t.ry0 = r[1];
+      t.rx1 = r[2];
+      t.ry1 = r[3];
+      t.inst = s->ninst ? (int)k : -1;
+      bool any = false;
+      for (int yy = t.y0; yy < t.y1 && !any; yy++)
+        for (int xx = t.x0; xx < t.x1 && !any; xx++) any = cls[(size_t)yy * pitch + xx] != 0;
+      if (!any) return false;
+      bool plain = x - h >= r[0] && y - h >= r[1] && t.x1 + h <= r[2] && t.y1 + h <= r[3] &&
+                   (only_plain || sh.rx == sh.plain_rx);
+      for (int yy = y - h; yy < t.y1 + h && plain; yy++)
+        for (int xx = x - h; xx < t.x1 + h && plain; xx++)
+          plain = cls[(size_t)yy * pitch + xx] == 1;
+      if (only_plain && !plain) return false;
+      t.plain = plain ? 1 : 0;
+      s->lds_all.push_back(t);
+      return true;
+    };
     for (int y = r[1] + 1; y < r[3] - 1; y += bh)
-      for (int x = r[0] + 1; x < r[2] - 1; x += bw) {
-        LdsTile t;
-        t.x0 = x;
-        t.y0 = y;
-        t.x1 = std::min(x + bw, r[2] - 1);
-        t.y1 = std::min(y + bh, r[3] - 1);
-        t.rx0 = r[0];
-        t.ry0 = r[1];
-        t.rx1 = r[2];
-        t.ry1 = r[3];
-        t.inst = s->ninst ? (int)k : -1;
-        bool any = false;
-        for (int yy = t.y0; yy < t.y1 && !any; yy++)
-          for (int xx = t.x0; xx < t.x1 && !any; xx++) any = cls[(size_t)yy * pitch + xx] != 0;
-        if (!any) continue;
-        bool plain = x - h >= r[0] && y - h >= r[1] && t.x1 + h <= r[2] && t.y1 + h <= r[3];
-        for (int yy = y - h; yy < t.y1 + h && plain; yy++)
-          for (int xx = x - h; xx < t.x1 + h && plain; xx++)
-            plain = cls[(size_t)yy * pitch + xx] == 1;
-        t.plain = plain ? 1 : 0;
-        s->lds_all.push_back(t);
+      for (int x = r[0] + 1; x < r[2] - 1; x += pw) {
+        if (pw != bw && add(x, y, pw, true)) continue;
+        for (int xs = x; xs < std::min(x + pw, r[2] - 1); xs += bw)
+          add(xs, y, std::min(bw, x + pw - xs), false);
       }
   }
   if (s->lds_all.empty()) return LBM_OK;

@@ -67,6 +67,17 @@ def test_channels(prec, coll, nx, ny, d, extra):
             **extra)
 
 
+@pytest.mark.parametrize("coll", [lbm.BGKW, lbm.TRT, lbm.MRT])
+@pytest.mark.parametrize("nx,ny", [(621, 660), (905, 898)])
+def test_wide_fp64_blocks(coll, nx, ny):
+    """Blocks of 64 x 32 nodes in registers beside 32 x 32 ones: an obstacle
+    inside, sides that leave a part of a wide block."""
+    print("lds wide", coll, nx, ny, flush=True)
+    compare(lbm.Case.cavity_ex(nx, ny, [(300, 200, 355, 231)]), (21, 3, 2, 9), collision=coll,
+            precision=lbm.PREC_F64, uavg=0.1, viscosity=0.04, trt_lambda=0.25, trt_fp64_parts=1,
+            resid_kind=lbm.RESID_NONE)
+
+
 def test_fp32_bgk_with_two_step_launches_keeps_them():
     """Its two-step kernel rounds differently from the single step: the fields
     stay those of these launches."""
