@@ -97,9 +97,11 @@ __device__ inline R lane_pull(R x) {
 // nodes, and a third of the LDS accesses is left for two nodes per thread, a
 // sixth for four: FP64 BGK 4097^2 146.5 -> 130.6 us per step, 2049^2 40.2 ->
 // 37.0, 1025^2 11.2 -> 9.9; there memory and VALU issue bound it together
-// (34 bytes per node and step: 4.4 TB/s).  FP32 and FP16 keep the LDS form: the
-// DPP moves are VALU instructions, which bound them (FP32 MRT 4097^2 63.2
-// against 68.8 us).
+// (34 bytes per node and step: 4.4 TB/s).  For FP32 and FP16 the same form at
+// 32 x 32 with three workgroups per CU is the faster one up to 1.7 M and 3 M
+// cells (FP32 MRT 970^2 6.4 -> 5.7 us); above, the DPP moves, which are VALU
+// instructions, cost more than they save (FP32 MRT 4097^2 63.2 us against
+// 68.8).  Eight and six nodes per thread were 20-40 % slower there.
 // Ordinary stores: two blocks store parts of a cache line where they meet,
 // and non-temporal stores gave those to memory one by one (4097^2 FP32 82.7
 // against 63.2 us per step, FP64 165.6 against 144.8).

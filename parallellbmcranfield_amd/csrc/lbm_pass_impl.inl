@@ -60,7 +60,7 @@ static hipError_t lds_launch(const Launch& L) {
   };
   switch (L.lds_shape) {
     case 0: return go(k_lds_steps<S, COLL, 512, 32, 1, 1>, 512);
-    case 1: return go(k_lds_steps<S, COLL, 512, 32, 2, 4, 32, 2, !S::DEV>, 512);
+    case 1: return go(k_lds_steps<S, COLL, 512, 32, 2, S::DEV ? 6 : 4, 32, 2, true>, 512);
     case 3:  // TRT at 128 VGPRs spills (2049^2 74.8 us per step)
       if constexpr (!S::DEV && COLL != 2)
         return go(k_lds_steps<S, COLL, 512, 32, 2, 4, 64, 4, true>, 512);

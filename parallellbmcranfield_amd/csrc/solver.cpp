@@ -355,24 +355,36 @@ static int rebuild_lds_tiles(lbm_solver* s) {
 
 // Region shape and halo (a launch makes at most halo + 1 steps), by the
 // lattice's size.  Small lattices are bound by the latency of a launch and of
-// its steps: small regions, as many workgroups as CUs, and as many steps per
-// launch as still leave a few rows of output.  From a few hundred thousand
-// cells the chip is full and the nodes formed more than once weigh most:
-// larger regions and fewer steps, fewest where a step moves least (FP16) or
-// a node costs most (stochastic rounding).  FP64 keeps 32 x 32 in LDS (64 x 32
-// leaves one workgroup per CU) and takes 64 x 32 in registers for blocks of
-// interior nodes: BGK 700^2 7.1 -> 6.2 at halo 3 (7.6 at 4), 1025^2 11.2 -> 9.9
-// at halo 4 (10.7 at 3 and 5), 2049^2 40.2 -> 37.0, 4097^2 146.5 -> 130.6; MRT
-// 2049^2 45.2 -> 39.8.  TRT needs more registers than two workgroups leave and
-// stays at 32 x 32 (46.2 -> 44.8).  Measured, us per step, regions 32 x 16 /
-// 32 x 32 / 64 x 32 at their best halo: FP64 BGK 129^2 1.50 / 2.88 / 4.1,
-// 361^2 2.75 / 3.5 / -, 725^2 7.9 / 7.7 / -, 1025^2 13.2 / 12.7 / 14.7; FP32
-// MRT 129^2 1.20 / 1.96 / 2.8, 361^2 1.91 / 2.38 / 2.9, 725^2 4.98 / 4.65 /
-// 4.42, 1025^2 8.8 / 7.9 / 6.7; FP16 BGK 725^2 3.89 / 3.99 / 4.18, 1449^2 - /
-// 11.4 / 10.3.  Packed lattices, whose many walls weigh more in larger
-// regions: 48 cavities, 1.3 M nodes, FP32 14.1 / 12.5 / 13.3.
+// its steps: small regions in LDS, as many workgroups as CUs, and as many steps
+// per launch as still leave a few rows of output.  From 400 000 cells the chip
+// is full and the nodes formed more than once weigh most: 32 x 32 regions, with
+// blocks of interior nodes in registers, and fewer steps, fewest where a step
+// moves least (FP16) or a node costs most (stochastic rounding).  The largest
+// FP32 and FP16 lattices take 64 x 32 regions in LDS: fewer bytes, and no DPP
+// moves where VALU issue is short.  FP64, whose LDS form allows only 32 x 32,
+// takes 64 x 32 in registers; TRT needs more registers than two workgroups
+// leave and stays at 32 x 32.  Measured, us per step:
+//   32 x 16 in LDS / 32 x 32 in registers: FP32 MRT 360^2 1.93 / 2.39, 450^2
+//   2.51 / 2.77; FP16 MRT 650^2 3.95 / 3.82, BGK 500^2 2.55 / 2.74; FP64 MRT
+//   560^2 5.6 / 5.7; stochastic rounding BGK 850^2 6.7 / 7.0
+//   64 x 32 in LDS / 32 x 32 in registers: FP32 MRT 700^2 4.4 / 3.8, 970^2 6.4
+//   / 5.7, 1160^2 7.7 / 7.0, 1340^2 9.3 / 9.3; FP16 BGK 900^2 5.65 / 5.10,
+//   1300^2 8.3 / 7.8, 1600^2 11.3 / 11.0, 2500^2 23.05 / -; stochastic rounding
+//   TRT 1300^2 13.9 / 12.6
+//   FP64 BGK 32 x 32 in LDS / 64 x 32 in registers: 700^2 7.1 / 6.2 at halo 3
+//   (7.6 at 4), 1025^2 11.2 / 9.9 at halo 4 (10.7 at 3 and 5), 2049^2 40.2 /
+//   37.0, 4097^2 146.5 / 130.6; MRT 2049^2 45.2 / 39.8; TRT 2049^2, 32 x 32,
+//   46.2 / 44.8
+// Packed lattices, whose many walls weigh more in larger regions: 48 cavities,
+// 1.3 M nodes, FP32, 1000 steps and their evaluations: 32 x 32 in LDS 11.9 ms,
+// in registers 11.5 (halo 3).
 static void pick_lds_shape(lbm_solver* s, long long cells) {
-  const bool f64 = s->prec == LBM_PREC_F64, sr = s->prec == LBM_PREC_F16_SR;
+  const bool f64 = s->prec == LBM_PREC_F64, f32 = s->prec == LBM_PREC_F32,
+             sr = s->prec == LBM_PREC_F16_SR;
+  const lbm_options& o = s->opt;
+  int run = 0;  // plain steps between sampled ones (0: none are sampled)
+  if (o.resid_kind == LBM_RESID_FULL || o.resid_kind == LBM_RESID_VELOCITY) run = o.resid_every - 1;
+  if (o.force_id != 0 && o.force_every > 0 && (run == 0 || o.force_every < run)) run = o.force_every;
   if (cells < 25000) {
     s->lds_shape = 0;
     s->lds_halo = 6;
@@ -385,12 +397,18 @@ static void pick_lds_shape(lbm_solver* s, long long cells) {
   } else if (f64 && !s->ninst && s->coll != LBM_TRT) {
     s->lds_shape = 3;
     s->lds_halo = cells < 800000 ? 3 : 4;
-  } else if (f64 || (s->ninst && !sr)) {
+  } else if (f64) {
     s->lds_shape = 1;
     s->lds_halo = 4;
+  } else if ((s->ninst && !sr) || cells < (f32 ? 1700000 : 3000000)) {
+    s->lds_shape = 1;
+    s->lds_halo = f32 || (!sr && (s->ninst || cells < 1500000)) ? 3 : 2;
+    // runs that sampled steps cut short of whole launches
+    auto fill = [&](int per) { return (double)run / ((run + per - 1) / per * per); };
+    if (s->lds_halo == 3 && run > 0 && fill(4) < 0.9 && fill(5) > fill(4)) s->lds_halo = 4;
   } else {
     s->lds_shape = 2;
-    s->lds_halo = s->prec == LBM_PREC_F32 ? (cells < 900000 ? 5 : 4) : 3;
+    s->lds_halo = f32 ? 4 : 3;
   }
 }
 

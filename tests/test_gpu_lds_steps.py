@@ -78,6 +78,19 @@ def test_wide_fp64_blocks(coll, nx, ny):
             resid_kind=lbm.RESID_NONE)
 
 
+@pytest.mark.parametrize("prec", [lbm.PREC_F32, lbm.PREC_F16, lbm.PREC_F16_SR])
+@pytest.mark.parametrize("coll", [lbm.BGKW, lbm.TRT, lbm.MRT])
+@pytest.mark.parametrize("nx,ny", [(640, 631), (905, 898), (1290, 1270), (1745, 1731)])
+def test_low_precision_blocks_in_registers(prec, coll, nx, ny):
+    """The sizes around which the block shapes change; a residual cuts the runs."""
+    if coll == lbm.BGKW and prec == lbm.PREC_F32 and nx > 1000:
+        pytest.skip("takes two-step launches")
+    print("lds registers", prec, coll, nx, ny, flush=True)
+    compare(lbm.Case.cavity_ex(nx, ny, [(300, 200, 355, 231)]), (23, 3), collision=coll,
+            precision=prec, uavg=0.1, viscosity=0.04, trt_lambda=0.25, trt_fp64_parts=1,
+            resid_kind=lbm.RESID_VELOCITY, resid_every=10)
+
+
 def test_fp32_bgk_with_two_step_launches_keeps_them():
     """Its two-step kernel rounds differently from the single step: the fields
     stay those of these launches."""
