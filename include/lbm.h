@@ -141,7 +141,8 @@ typedef struct lbm_options {
  * LBM_TUNE_NO_TWO_STEP: every step its own launch.  By default runs of plain
  * steps go several to a launch with each block of nodes held in LDS between
  * them (lbm_solver_fused reports how many), on every lattice without open
- * outlets; the last step of a call is a single one.  Captured graphs, split
+ * outlets but FP32 BGK ones with two-step launches, whose rounding differs;
+ * the last step of a call is a single one.  Captured graphs, split
  * launches and two_step_rows or three_step_rows > 0 turn that off.
  * Two plain steps in a row also run as one pass over the state where that
  * pays for runs too short for the above (FP32

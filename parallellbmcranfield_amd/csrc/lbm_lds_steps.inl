@@ -86,12 +86,13 @@ __device__ inline R lane_pull(R x) {
 // reads, the collision's dependent chain, two barriers); 129^2 FP64 BGK 4.12
 // us per single-step launch, 1.50 us per step at seven a launch.  Large
 // lattices: VALU issue and memory together.  A block of 64 x 32 nodes makes
-// five steps of 56 x 24, forming 1.37 nodes per node kept and reading 1.67
+// five steps of 56 x 24, forming 1.37 nodes per node kept and reading 1.52
 // times what it keeps, where k_three_steps reads 1.72 times the state per
 // three steps and two-step launches as much per two: 4097^2 FP32 MRT 115.2 ->
-// 63.2 us per step (145 -> 265 GLUPS), 2049^2 39.7 -> 19.2, 1025^2 15.2 -> 7.0;
-// FP64 BGK 4097^2 274 -> 145, 2049^2 72 -> 39; FP16 BGK 4097^2 111.8 -> 56.4.
-// LANES (FP64): 72 bytes of LDS per node and step's 18 accesses limited FP64
+// 63.2 us per step (145 -> 265 GLUPS), 2049^2 39.7 -> 19.2, 1025^2 15.2 -> 7.0
+// (6.5 with LANES); FP64 BGK 4097^2 274 -> 145 (130 with LANES), 2049^2 72 -> 39
+// (37); FP16 BGK 4097^2 111.8 -> 56.4.
+// LANES: 72 bytes of LDS per node and step's 18 accesses limited FP64
 // to regions of 32 x 32, which form 1.69 nodes per node kept and read 1.78.
 // Blocks of interior nodes now hold their state in registers, a wave 64 x 4
 // nodes, and a third of the LDS accesses is left for two nodes per thread, a
