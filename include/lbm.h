@@ -275,12 +275,12 @@ int lbm_solver_step(lbm_solver* s, int nsteps, int* done);
 /* Same, timing the step kernel with HIP events on the solver's stream around
  * every `sample_every`-th launch (1 = every launch).  total_ms: stream time of
  * the nsteps; kernel_ms: average duration of one sampled step-kernel launch.
- * With LDS-resident blocks (lbm_solver_fused) the sampled kernel is theirs,
- * up to that many steps per launch.  With two- or three-step launches alone
- * (lbm_solver_two_step_info, lbm_solver_three_step_info) it is the three-step
- * kernel (one launch per three steps) where three-step launches are on, else
- * the two-step kernel (one launch per two steps); launches of fewer steps
- * are not sampled. */
+ * Where launches of several kernels were sampled, it is the average of one
+ * kernel's: that of the LDS-resident blocks (lbm_solver_fused; up to that many
+ * steps per launch) if the call made such launches, else the three-step
+ * kernel's, else the two-step kernel's (one launch per three or two steps;
+ * lbm_solver_three_step_info, lbm_solver_two_step_info), else the single
+ * step's. */
 int lbm_solver_step_timed(lbm_solver* s, int nsteps, int sample_every, double* total_ms,
                           double* kernel_ms);
 int lbm_solver_sync(lbm_solver* s);

@@ -1685,10 +1685,15 @@ static int batch_eval(lbm_solver* s) {
   return LBM_OK;
 }
 
-// evs: timing events, two per sample; rec receives the event-pair index of
-// every sample taken.
+// A launch of a timed call: its kernel, and the first of its two events.
+struct Sampled {
+  enum Kernel { SINGLE, TWO, THREE, LDS } kernel;
+  size_t ei;
+};
+
+// evs: timing events, two per sample; rec receives every sample taken.
 static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_t>* evs,
-                     int sample_every = 1, std::vector<size_t>* rec = nullptr) {
+                     int sample_every = 1, std::vector<Sampled>* rec = nullptr) {
   if (s->ninst && s->t_first_step < 0) s->t_first_step = wall_seconds();
   if (done) *done = 0;
   if (s->invalid) {
@@ -1786,7 +1791,7 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
         int rc = launch_lds_steps(s, s->cur, k, sample ? (*evs)[ei] : nullptr,
                                   sample ? (*evs)[ei + 1] : nullptr);
         if (rc) return rc;
-        if (sample && rec) rec->push_back(ei);
+        if (sample && rec) rec->push_back({Sampled::LDS, ei});
         s->cur ^= 1;
         made(k);
         t += k - 1;
@@ -1811,7 +1816,7 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
         const size_t ei = 2 * (size_t)(ts / sample_every);
         int rc = launch_three_steps(s, s->cur, (*evs)[ei], (*evs)[ei + 1]);
         if (rc) return rc;
-        if (rec) rec->push_back(ei);
+        if (rec) rec->push_back({Sampled::THREE, ei});
       } else if (s->use_graph) {
         if (!s->gexec3[s->cur]) {  // both parities at once: the other is next
           int rc = build_graph3(s, s->cur);
@@ -1832,11 +1837,11 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
     }
     // Two plain steps in a row with two-step launches: one pass over the state.
     if (s->two && plain_pair) {
-      if (sample_pair && !s->three) {  // with three-step launches only those are sampled
+      if (sample_pair) {
         const size_t ei = 2 * (size_t)((t % sample_every == 0 ? t : t + 1) / sample_every);
         int rc = launch_two_steps(s, s->cur, (*evs)[ei], (*evs)[ei + 1]);
         if (rc) return rc;
-        if (rec) rec->push_back(ei);
+        if (rec) rec->push_back({Sampled::TWO, ei});
       } else if (s->use_graph) {
         if (!s->gexec2[s->cur]) {  // both parities at once
           int rc = build_graph2(s, s->cur);
@@ -1873,12 +1878,10 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
     L.kp.res_kind = rpart ? (rk == LBM_RESID_FULL ? RK_FULL : RK_VEL) : RK_NONE;
     L.kp.force_on = feval ? 1 : 0;
     if (rk == LBM_RESID_REFERENCE) L.out.cres = s->d_cres;
-    // with multi-step launches only those are sampled (runs too short for one aside)
-    const bool timed = evs && !s->two && !s->three && (!s->lds || nsteps < 3) &&
-                       (t % sample_every == 0);
+    const bool timed = evs && (t % sample_every == 0);
     const size_t ei = 2 * (size_t)(t / (sample_every > 0 ? sample_every : 1));
     if (timed) HC(hipEventRecord((*evs)[ei], s->stream));
-    if (timed && rec) rec->push_back(ei);
+    if (timed && rec) rec->push_back({Sampled::SINGLE, ei});
     if (s->fused) {
       HC(pass(s, mode, PASS_FUSED, L));  // bulk tiles + boundary-list nodes, one launch
       if (timed) HC(hipEventRecord((*evs)[ei + 1], s->stream));
@@ -1940,17 +1943,22 @@ int lbm_solver_step_timed(lbm_solver* s, int nsteps, int sample_every, double* t
   hipEvent_t e0 = s->ev[2 * nsamp], e1 = s->ev[2 * nsamp + 1];
   HC(hipEventRecord(e0, s->stream));
   int done = 0;
-  std::vector<size_t> rec;
+  std::vector<Sampled> rec;
   int rc = step_impl(s, nsteps, &done, &evs, sample_every, &rec);
   HC(hipEventRecord(e1, s->stream));
   HC(hipEventSynchronize(e1));
   float ms = 0.f;
   HC(hipEventElapsedTime(&ms, e0, e1));
+  // the kernel of the most steps among those that ran: a call whose steps are
+  // all evaluated makes single-step launches alone
+  Sampled::Kernel most = Sampled::SINGLE;
+  for (const Sampled& r : rec) most = std::max(most, r.kernel);
   double bsum = 0.0;
   int nb = 0;
-  for (size_t ei : rec) {
+  for (const Sampled& r : rec) {
+    if (r.kernel != most) continue;
     float b = 0.f;
-    HC(hipEventElapsedTime(&b, evs[ei], evs[ei + 1]));
+    HC(hipEventElapsedTime(&b, evs[r.ei], evs[r.ei + 1]));
     bsum += b;
     nb++;
   }
