@@ -288,11 +288,8 @@ def main():
     t1 = time.perf_counter()
     wall = t1 - t0
     nf = case.info.num_fluid
-    n_bulk, steps_per_launch, kname = timed_kernel(s, case)
-    lds = s.lds_steps > 0
-    sampled = timed_launches(args.steps, args.sample_every, steps_per_launch, lds)
-    if lds and sampled:
-        steps_per_launch = round(sum(sampled) / len(sampled), 4)
+    n_bulk, sampled, kname = timed_kernel(s, case, args.steps, args.sample_every)
+    steps_per_launch = mean_steps(sampled)
     two = s.two_step_info()
     three = s.three_step_info()
     mlups = nf * args.steps / wall / 1e6
@@ -313,7 +310,8 @@ def main():
     if default_shape and os.path.exists(PMC_SUMMARY):
         try:
             pm = json.load(open(PMC_SUMMARY))
-            prefix = "lds_" if lds else {1: "", 2: "two_", 3: "three_"}[steps_per_launch]
+            prefix = {"k_lds_steps": "lds_", "k_three_steps": "three_",
+                      "k_two_steps": "two_"}.get(kname.split()[0], "")
             key = f"{prefix}{args.collision}_{args.precision}_{N}"
             if key in pm.get("kernels", {}):
                 traffic = pm["kernels"][key]["hbm_bytes_per_launch"]
@@ -333,9 +331,8 @@ def main():
         o64 = lbm.make_options(**kw)
         o64.precision = lbm.PREC_F64
         s64 = lbm.Solver(case, o64)
-        n64, spl64, _ = timed_kernel(s64, case)
-        made = timed_launches(args.steps, args.sample_every, spl64, s64.lds_steps > 0)
-        spl64 = round(sum(made) / max(len(made), 1), 4) if s64.lds_steps else spl64
+        n64, made, _ = timed_kernel(s64, case, args.steps, args.sample_every)
+        spl64 = mean_steps(made)
         s64.step(args.warmup)
         s64.sync()
         t0 = time.perf_counter()
@@ -430,18 +427,17 @@ def main():
     print(json.dumps(out), flush=True)
 
 
-def timed_launches(steps: int, every: int, per_launch: int, lds: bool) -> list[int]:
-    """Steps made by each launch lbm_solver_step_timed brackets with events in
-    a run of plain steps: those that hold every `every`-th step.  Two- and
-    three-step launches make exactly as many (a run's last steps may take a
-    launch of fewer, which is not sampled); LDS-resident ones at most
-    per_launch, the last two of a run sharing what is left, and the last step
-    of a call is a single one."""
+def timed_launches(steps: int, every: int, per_launch: int, lds: bool, least: int = 2) -> list[int]:
+    """Steps made by each launch of one kernel that lbm_solver_step_timed
+    samples in a run of plain steps: those that hold every `every`-th step.
+    Two- and three-step launches make exactly as many; LDS-resident ones
+    `least` to per_launch, the last two of a run sharing what is left, and the
+    last step of a call is not theirs."""
     if per_launch == 1:
         return [1] * ((steps + every - 1) // every)
     made, t = [], 0
     end = steps - 1 if lds else steps
-    while end - t >= (2 if lds else per_launch):
+    while end - t >= (least if lds else per_launch):
         left = end - t
         k = per_launch
         if lds and left < 2 * per_launch - 1:
@@ -452,29 +448,43 @@ def timed_launches(steps: int, every: int, per_launch: int, lds: bool) -> list[i
     return made
 
 
-def timed_kernel(s, case):
-    """The kernel lbm_solver_step_timed samples: nodes one launch updates,
-    steps per launch and its name.  Three-step launches: the three-step
-    tiles' nodes, three steps; two-step launches: the two-step tiles' nodes,
-    two steps (the band's single steps are separate launches); else the fused
-    step kernel (bulk tiles and boundary-list nodes; FP16: its paired-cell
-    form) or the bulk kernel.  With LDS-resident blocks, which come first, every
-    fluid node and the most steps a launch makes."""
+def timed_kernel(s, case, steps: int, every: int):
+    """The kernel whose launches lbm_solver_step_timed averages over a run of
+    `steps` plain steps: nodes one launch updates, the steps of each sampled
+    launch, and its name.  With LDS-resident blocks, which come first where
+    the run is long enough for one, every fluid node.  Three-step launches:
+    the three-step tiles' nodes; two-step launches: the two-step tiles' nodes
+    (the band's single steps are separate launches); else the fused step
+    kernel (bulk tiles and boundary-list nodes; FP16: its paired-cell form) or
+    the bulk kernel."""
+    three, two = s.three_step_info(), s.two_step_info()
     if s.lds_steps:
-        return (case.info.num_fluid, s.lds_steps,
-                "k_lds_steps (runs of plain steps with LDS-resident blocks)")
-    three = s.three_step_info()
+        # from 2^22 cells lattices with two- or three-step launches leave runs of two to those
+        least = 3 if (two["cells"] or three["cells"]) and case.n * case.m >= 1 << 22 else 2
+        made = timed_launches(steps, every, s.lds_steps, True, least)
+        if made:
+            return (case.info.num_fluid, made,
+                    "k_lds_steps (runs of plain steps with LDS-resident blocks)")
     if three["cells"] > 0:
-        return three["cells"], 3, "k_three_steps (three steps per launch over the three-step tiles)"
-    two = s.two_step_info()
+        made = timed_launches(steps, every, 3, False)
+        if made:
+            return (three["cells"], made,
+                    "k_three_steps (three steps per launch over the three-step tiles)")
     if two["cells"] > 0:
-        return two["cells"], 2, "k_two_steps (two steps per launch over the two-step tiles)"
+        made = timed_launches(steps, every, 2, False)
+        if made:
+            return two["cells"], made, "k_two_steps (two steps per launch over the two-step tiles)"
+    made = timed_launches(steps, every, 1, False)
     nf = case.info.num_fluid
     if s.paired:
-        return nf, 1, "k_step_pair (FP16, two cells per thread; bulk tiles + boundary-list nodes)"
+        return nf, made, "k_step_pair (FP16, two cells per thread; bulk tiles + boundary-list nodes)"
     if s.fused:
-        return nf, 1, "k_step (bulk tiles + boundary-list nodes)"
-    return nf - case.info.num_boundary, 1, "k_bulk"
+        return nf, made, "k_step (bulk tiles + boundary-list nodes)"
+    return nf - case.info.num_boundary, made, "k_bulk"
+
+
+def mean_steps(made: list[int]) -> float:
+    return round(sum(made) / max(len(made), 1), 4)
 
 
 def bench_sweep(args):
@@ -795,7 +805,8 @@ def bench_cavity129(args):
                           init=lbm.INIT_REST, resid_kind=lbm.RESID_NONE, use_stop_rule=0)
     o2.precision = lbm.PREC_F64
     s2 = lbm.Solver(case, o2)
-    nl, spl, _ = timed_kernel(s2, case)
+    nl, made, _ = timed_kernel(s2, case, 2000, 8)
+    spl = mean_steps(made)
     s2.step(50)
     _, kern_ms = s2.step_timed(2000, 8)
     s2.close()
@@ -873,10 +884,8 @@ def bench_matrix(args):
                 o = lbm.make_options(**kw)
                 o.precision = prec
                 s = lbm.Solver(case, o)
-                nl, spl, _ = timed_kernel(s, case)
-                if s.lds_steps:
-                    made = timed_launches(args.steps, args.sample_every, spl, True)
-                    spl = round(sum(made) / max(len(made), 1), 4)
+                nl, made, _ = timed_kernel(s, case, args.steps, args.sample_every)
+                spl = mean_steps(made)
                 s.step(args.warmup)
                 s.sync()
                 t0 = time.perf_counter()
