@@ -170,7 +170,8 @@ def autotune(case: Case, opts, instances=None, steps: int = 198,
     launches: two plain steps per launch with `two_rows` output rows per
     256-column tile, three per launch with `three_rows` (single lattices
     only; 0: the library's own pick, runs of steps with LDS-resident blocks
-    where it has them), each against single steps.  A variant whose
+    where it has them), each against single steps; and that pick at block
+    256, the only one with such runs, whatever won stage 1.  A variant whose
     solver runs no such launches is dropped.  `best` holds the options to
     copy (block_size, xcd_group, two_step_rows, three_step_rows, tune_flags)
     and what ran."""
@@ -208,6 +209,15 @@ def autotune(case: Case, opts, instances=None, steps: int = 198,
                 results.append(record(o, dt, two, three, 1))
     best1 = min(results, key=lambda r: r["ms_per_step"])
     base = best1["tune_flags"] & ~single
+    # Runs of steps with LDS-resident blocks exist at block 256 alone, where
+    # they are worth two to three times more than any stage-1 shape.
+    best256 = min((r for r in results if r["block_size"] == 256),
+                  key=lambda r: r["ms_per_step"], default=None)
+    if best256 and not (best256 is best1 and 0 in two_rows):
+        o = variant(256, best256["xcd_group"], best256["tune_flags"] & ~single)
+        dt, two, three = _time_steps(case, o, instances, steps)
+        if two.get("lds_steps"):
+            results.append(record(o, dt, two, three, 2))
     for r2 in two_rows:
         o = variant(best1["block_size"], best1["xcd_group"], base | TUNE_NO_THREE_STEP, rows2=r2)
         dt, two, three = _time_steps(case, o, instances, steps)
