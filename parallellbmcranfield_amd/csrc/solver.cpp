@@ -35,7 +35,9 @@ static int launch_step_passes(lbm_solver* s, const Launch& L);
 
 namespace {
 
-constexpr int HCAP = 1024;  // history slots
+// History slots: they are read once HCAP are taken; a force pass and the step
+// after it may each take one more.
+constexpr int HCAP = 1024;
 constexpr int HW = 8;       // slot: raw residual [0..3], force [4..5], unused [6..7]
 
 int dev_alloc(lbm_solver* s, void** p, size_t bytes) {
@@ -1111,10 +1113,10 @@ static int solver_create(const lbm_case* c, const lbm_options* o, const double* 
   // the kernels write their sums where the host reads them: no copy behind an
   // evaluation, only the wait
   if (!rc)
-    rc = check_hip(hipHostMalloc((void**)&s->hist, sizeof(double) * (HW * HCAP + 2 * (size_t)ninst),
+    rc = check_hip(hipHostMalloc((void**)&s->hist, sizeof(double) * (HW * (HCAP + 1) + 2 * (size_t)ninst),
                                  hipHostMallocDefault),
                    "residual rows");
-  if (!rc) s->inst_raw = s->hist + HW * HCAP;
+  if (!rc) s->inst_raw = s->hist + HW * (HCAP + 1);
   if (!rc && s->prec == LBM_PREC_F16_SR) {  // step number of stochastic rounding, 2 slots
     rc = dev_alloc(s, (void**)&s->d_seed, 2 * sizeof(uint32_t));
     if (!rc) rc = check_hip(hipMemset(s->d_seed, 0, 2 * sizeof(uint32_t)), "clear step number");
@@ -1746,16 +1748,13 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
                       : launch_pass_lp(s->prec, 1, MODE_RESID, PASS_FORCE, L));
       s->pending_iter.push_back(s->iter);
       s->pending_what.push_back(2);
-      if (++s->pending == HCAP) {
-        int rc = flush_history(s);
-        if (rc) {
-          if (done) *done = ran;
-          return rc;
-        }
-      }
+      s->pending++;
     }
     const bool feval = !s->force_pass && forces_at(s->iter);
-    const bool eval = reval || feval;
+    // The history is read after a single step: a divergence that it shows ends
+    // the call there, with the state one step back in buf[cur^1].
+    const bool full = s->pending >= HCAP;
+    const bool eval = reval || feval || full;
     // The stop rule reads only evaluated residuals, which change at
     // evaluation steps alone, and a run of plain steps holds none: the rule
     // cannot end the run inside it, so runs of two- and three-step launches
@@ -1910,7 +1909,7 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
         return rc;
       }
     }
-    if (s->pending == HCAP || (reval && stop_can_trigger)) {
+    if (s->pending >= HCAP || (reval && stop_can_trigger)) {
       int rc = flush_history(s);
       if (rc) {
         if (done) *done = ran;

@@ -1,0 +1,41 @@
+"""A history that fills inside a call: where it shows a divergence the call ends
+with the fields of the iteration it reports, whatever launches came before."""
+import numpy as np
+import pytest
+
+import parallellbmcranfield_amd as lbm
+
+pytestmark = pytest.mark.gpu
+
+NX, NY = 5000, 20
+
+
+def solver(resid, flags=0):
+    case = lbm.Case.channel(NX, NY, 50.2, 10.3, 4.0)
+    rho, u, v = np.ones((case.m, case.n)), np.zeros((case.m, case.n)), np.zeros((case.m, case.n))
+    u[10, NX - 10] = np.nan  # spreads by at most one node per step: most of the channel stays finite
+    return lbm.Solver(case, lbm.make_options(
+        rho_ini=1.0, init=lbm.INIT_FIELD, use_stop_rule=0, collision=lbm.BGKW,
+        precision=lbm.PREC_F64, uavg=0.03, viscosity=0.03, force_id=5, force_every=2,
+        resid_kind=resid, resid_every=500, curved=1, inlet_profile=1, outlet_profile=4,
+        tune_flags=flags), field=(rho, u, v))
+
+
+@pytest.mark.parametrize("flags", [0, lbm.TUNE_NO_TWO_STEP | lbm.TUNE_NO_THREE_STEP])
+def test_fields_after_a_divergence_are_those_of_its_iteration(flags):
+    print("full history", flags, flush=True)
+    s = solver(lbm.RESID_FULL, flags)
+    assert (s.lds_steps > 0) == (flags == 0)
+    with pytest.raises(lbm.LbmError) as e:
+        s.step(4000)
+    assert e.value.code == lbm.DIVERGED
+    # 1024 rows: the forces of every second step, the residuals of 500, 1000, 1500 and 2000
+    assert s.iter == 2 * 1020
+    got = s.macro()
+    s.close()
+    s = solver(lbm.RESID_NONE, lbm.TUNE_NO_TWO_STEP | lbm.TUNE_NO_THREE_STEP)
+    s.step(2 * 1020)
+    want = s.macro()
+    s.close()
+    assert np.isnan(want[1]).any() and np.isfinite(want[1]).mean() > 0.5
+    assert all(np.array_equal(x, y, equal_nan=True) for x, y in zip(got, want))
