@@ -386,7 +386,11 @@ static void pick_lds_shape(lbm_solver* s, long long cells) {
   const lbm_options& o = s->opt;
   int run = 0;  // plain steps between sampled ones (0: none are sampled)
   if (o.resid_kind == LBM_RESID_FULL || o.resid_kind == LBM_RESID_VELOCITY) run = o.resid_every - 1;
-  if (o.force_id != 0 && o.force_every > 0 && (run == 0 || o.force_every < run)) run = o.force_every;
+  if (o.force_id != 0 && o.force_every > 0) {
+    // a force step opens a run, or is a residual step and ends one
+    const int frun = s->force_pass ? o.force_every : o.force_every - 1;
+    if (run == 0 || frun < run) run = frun;
+  }
   if (cells < 25000) {
     s->lds_shape = 0;
     s->lds_halo = 6;
