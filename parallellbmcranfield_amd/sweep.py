@@ -170,9 +170,9 @@ def autotune(case: Case, opts, instances=None, steps: int = 198,
     launches: two plain steps per launch with `two_rows` output rows per
     256-column tile, three per launch with `three_rows` (single lattices
     only; 0: the library's own pick, runs of steps with LDS-resident blocks
-    where it has them), each against single steps; and that pick at block
-    256, the only one with such runs, whatever won stage 1.  A variant whose
-    solver runs no such launches is dropped.  `best` holds the options to
+    where it has them), each against single steps.  Block 256 is the only one
+    with such runs, so with 0 among `two_rows` it is timed whatever block won
+    stage 1.  A variant whose solver runs no such launches is dropped.  `best` holds the options to
     copy (block_size, xcd_group, two_step_rows, three_step_rows, tune_flags)
     and what ran."""
     from . import PREC_F16, PREC_F16_SR, TUNE_NO_PAIRS, TUNE_NO_THREE_STEP, TUNE_NO_TWO_STEP
@@ -213,7 +213,7 @@ def autotune(case: Case, opts, instances=None, steps: int = 198,
     # they are worth two to three times more than any stage-1 shape.
     best256 = min((r for r in results if r["block_size"] == 256),
                   key=lambda r: r["ms_per_step"], default=None)
-    if best256 and not (best256 is best1 and 0 in two_rows):
+    if best256 and best256 is not best1 and 0 in two_rows:
         o = variant(256, best256["xcd_group"], best256["tune_flags"] & ~single)
         dt, two, three = _time_steps(case, o, instances, steps)
         if two.get("lds_steps"):

@@ -8,7 +8,7 @@ from parallellbmcranfield_amd import sweep as SW
 
 @pytest.mark.parametrize("prec,instances", [(lbm.PREC_F32, None), (lbm.PREC_F16, None),
                                             (lbm.PREC_F32, [object()])])
-@pytest.mark.parametrize("rows", [(0,), (4,), (0, 4)])
+@pytest.mark.parametrize("rows", [(0,), (0, 4)])
 @pytest.mark.parametrize("winner", [256, 512])
 def test_the_default_launches_compete_whatever_block_wins_single_steps(monkeypatch, prec, instances,
                                                                        rows, winner):
@@ -30,15 +30,18 @@ def test_the_default_launches_compete_whatever_block_wins_single_steps(monkeypat
     assert sum(r["steps_per_launch"] == 5 for r in tried) == 1
 
 
-def test_blocks_without_256_are_taken_as_asked(monkeypatch):
+@pytest.mark.parametrize("blocks,rows", [((512,), (0,)), ((256, 512), (4,))])
+def test_blocks_and_rows_are_taken_as_asked(monkeypatch, blocks, rows):
+    """Without block 256, or without the library's own pick among the rows."""
     calls = []
 
     def timer(case, o, inst, steps):
-        calls.append(o.block_size)
+        calls.append((o.block_size, o.two_step_rows))
         tiles = dict(cells=0, tiles=0, rows=0, band=0)
-        return 1.0, dict(tiles, lds_steps=0), tiles
+        return 1.0 if o.block_size == 512 else 1.01, dict(tiles, lds_steps=0), tiles
 
     monkeypatch.setattr(SW, "_time_steps", timer)
     best, _ = SW.autotune(None, lbm.make_options(uavg=0.05, viscosity=0.03), steps=12,
-                          blocks=(512,), groups=(4,))
-    assert best["block_size"] == 512 and set(calls) == {512}
+                          blocks=blocks, groups=(4,), two_rows=rows)
+    assert best["block_size"] == 512
+    assert calls == [(b, 0) for b in blocks] + [(512, r) for r in rows] + [(512, 0)]
