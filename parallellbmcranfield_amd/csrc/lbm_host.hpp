@@ -91,7 +91,7 @@ struct lbm_solver {
   // row of it is zero, and no stop rule reads it: no step evaluates it
   bool ref_zero = false;
   double* d_part = nullptr;   // [nparts][4]
-  double* hist = nullptr;     // [HCAP + 1][8] sums of evaluations, pinned: kernels write, the host reads
+  double* hist = nullptr;     // [HSLOTS][8] sums of evaluations, pinned: kernels write, the host reads
   uint32_t* d_seed = nullptr; // FP16 stochastic rounding: step number, 2 slots
   int nparts = 0;
   int nb_bulk = 0, nb_bnd = 0, nb_out = 0;
