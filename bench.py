@@ -415,6 +415,9 @@ def main():
             "state_gbs": round(state_gbs, 1),
             "state_frac": round(state_gbs / HBM_PEAK_GBS, 4),
             "traffic_over_state": round(traffic / state_bytes_per_launch, 4) if traffic else None,
+            # what the counters say it moves: the share of the peak that is in use
+            "traffic_gbs": round(traffic / avg_bulk_s / 1e9, 1) if traffic else None,
+            "traffic_frac": round(traffic / avg_bulk_s / 1e9 / HBM_PEAK_GBS, 4) if traffic else None,
             "avg_launch_us": round(avg_bulk_s * 1e6, 2),
             "launches_timed": len(sampled),
             "copy_kernel_gbs": round(copy_gbs, 1),
