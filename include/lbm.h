@@ -141,9 +141,10 @@ typedef struct lbm_options {
  * LBM_TUNE_NO_TWO_STEP: every step its own launch.  By default runs of plain
  * steps go several to a launch with each block of nodes held in LDS between
  * them (lbm_solver_fused reports how many), on every lattice without open
- * outlets but FP32 BGK ones with two-step launches, whose rounding differs;
- * the last step of a call is a single one.  Captured graphs, split
- * launches and two_step_rows or three_step_rows > 0 turn that off.
+ * outlets but FP32 BGK ones with two-step launches, whose rounding differs,
+ * and FP16 ones with a scale that is no power of two; the last step of a call
+ * is not one of theirs.  Captured graphs, split launches, a block_size other
+ * than 256 and two_step_rows or three_step_rows > 0 turn that off.
  * Two plain steps in a row also run as one pass over the state where that
  * pays for runs too short for the above (FP32
  * storage on lattices of at least 2^20 cells, FP64 on lattices of at least

@@ -86,19 +86,26 @@ __device__ inline R lane_pull(R x) {
 // reads, the collision's dependent chain, two barriers); 129^2 FP64 BGK 4.12
 // us per single-step launch, 1.50 us per step at seven a launch.  Large
 // lattices: VALU issue and memory together.  A block of 64 x 32 nodes makes
-// five steps of 56 x 24, forming 1.37 nodes per node kept and reading 1.52
-// times what it keeps, where k_three_steps reads 1.72 times the state per
-// three steps and two-step launches as much per two: 4097^2 FP32 MRT 115.2 ->
-// 63.2 us per step (145 -> 265 GLUPS), 2049^2 39.7 -> 19.2, 1025^2 15.2 -> 7.0
-// (6.5 with LANES); FP64 BGK 4097^2 274 -> 145 (130 with LANES), 2049^2 72 -> 39
-// (37); FP16 BGK 4097^2 111.8 -> 56.4.
+// five steps of 56 x 24, forming 1.37 nodes per node kept and loading 1.52
+// times what it keeps (1.36 from memory, by the counters), where k_three_steps
+// reads 1.72 times the state per three steps and two-step launches 1.30 times
+// per two: 4097^2 FP32 MRT 115.2 -> 63.2 us per step (145 -> 265 GLUPS), 2049^2
+// 39.7 -> 19.2, 1025^2 15.2 -> 7.0 (6.5 with LANES); FP64 BGK 4097^2 274 -> 145
+// (130 with LANES), 2049^2 72 -> 39 (37); FP16 BGK 4097^2 111.8 -> 56.4.  Those
+// are runs from rest; on a developed field 4097^2 takes 69.5 (FP32), 139 (FP64
+// BGK) and 59.3 (FP16), 2049^2 FP64 38.5: as many cycles and instructions at a
+// lower clock (FP64 2.39 -> 2.21 GHz between iterations 500 and 5500).
+// Counters: 4097^2 FP32 0.77 M cycles per launch, whose VALU instructions fill
+// every issue slot of the SIMDs (104 % at four cycles each) beside 4.6 TB/s;
+// 1025^2 60 %, 2.9 TB/s.
 // LANES: 72 bytes of LDS per node and step's 18 accesses limited FP64
 // to regions of 32 x 32, which form 1.69 nodes per node kept and read 1.78.
 // Blocks of interior nodes now hold their state in registers, a wave 64 x 4
 // nodes, and a third of the LDS accesses is left for two nodes per thread, a
 // sixth for four: FP64 BGK 4097^2 146.5 -> 130.6 us per step, 2049^2 40.2 ->
 // 37.0, 1025^2 11.2 -> 9.9; there memory and VALU issue bound it together
-// (34 bytes per node and step: 4.4 TB/s).  For FP32 and FP16 the same form at
+// (2049^2, counters: 34 bytes per node and step, 3.9 TB/s; issue slots 61 %
+// full).  For FP32 and FP16 the same form at
 // 32 x 32 with three workgroups per CU is the faster one up to 1.7 M and 3 M
 // cells (FP32 MRT 970^2 6.4 -> 5.7 us); above, the DPP moves, which are VALU
 // instructions, cost more than they save (FP32 MRT 4097^2 63.2 us against

@@ -1774,11 +1774,15 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
     // lattice's launches are faster direct than replayed two to a graph (129^2
     // under its stop rule 8.1 against 5.7 us per step).
     // A run of plain steps with LDS-resident blocks.  The last step of a call
-    // (and the last before the iteration cap) is a single one, so that
-    // observe passes and checkpoints find the state one step back.  Runs of
-    // two on lattices with two- and three-step launches go to those (with the
-    // single step after them, us: 4097^2 FP32 403 for a three-step launch
-    // against 613, FP64 2049^2 254 against 317).
+    // (and the last before the iteration cap) is left to the launches below:
+    // a single step, after which observe passes and checkpoints find the state
+    // one step back.  Lattices with two- or three-step launches end a call
+    // with one of those where no longer run is left before it (two plain steps
+    // after an evaluation, or as a whole call; three from 2^22 cells), and
+    // observe passes then form the step in between again.  From 2^22 cells
+    // runs of two go to them too (with the single step after them, us: 4097^2
+    // FP32 403 for a three-step launch against 613, FP64 2049^2 254 against
+    // 317).
     if (s->lds && !eval) {
       const int most = s->lds_halo + 1;
       const int least = (s->two || s->three) && (long long)s->cs->n * s->cs->m >= (1LL << 22) ? 3 : 2;
