@@ -35,8 +35,8 @@ static int launch_step_passes(lbm_solver* s, const Launch& L);
 
 namespace {
 
-// History slots: they are read once all but one are taken, since a force pass
-// and the step after it may each take one.  64 kB: pinned allocations above that
+// History slots: they are read once all but one are taken, after the next
+// single step, which may take one too.  64 kB: pinned allocations above that
 // took 0.28 ms in place of 0.03 while others were held.
 constexpr int HSLOTS = 1024;
 constexpr int HCAP = HSLOTS - 1;
@@ -1236,8 +1236,12 @@ static int solver_create(const lbm_case* c, const lbm_options* o, const double* 
   // plain force step would move the fields by an ulp (FP32 BGK, 149 x 44
   // channel: 1e-5 of rho after 460 steps).  FP64 and MRT are the same bit for
   // bit in both forms.
-  const bool force_plain = s->prec == LBM_PREC_F64 || s->coll == LBM_MRT;
-  if (!rc && o->force_id != 0 && o->force_every > 0 && s->norows == 0 && s->fused && force_plain) {
+  // And so do forces of every step, which leave no run of plain steps: the
+  // residual form's force and reduction cost less than a launch of k_force
+  // (600 x 200, us per step: FP16 MRT 17.3 against 22.5, FP64 BGK 18.5 against
+  // 21.5; at every second step 15.8 against 8.3 and 15.4 against 10.0).
+  const bool force_plain = (s->prec == LBM_PREC_F64 || s->coll == LBM_MRT) && o->force_every > 1;
+  if (!rc && o->force_id != 0 && force_plain && s->norows == 0 && s->fused) {
     std::vector<int> body;
     for (size_t i = 0; i < bn.size(); i++)
       if (bn[i].boundary_id == o->force_id && (body.empty() || body.back() != (int)(i / 256)))
@@ -1747,7 +1751,9 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
     auto forces_at = [&](int it) {
       return o.force_id != 0 && o.force_every > 0 && (it + 1) % o.force_every == 0;
     };
-    if (s->force_pass && forces_at(s->iter)) {
+    // a step that is evaluated anyway takes the force along
+    const bool fpass = s->force_pass && !reval && forces_at(s->iter);
+    if (fpass) {
       Launch L = make_launch(s, s->cur);
       L.body = s->d_body;
       L.nbody = s->nbody;
@@ -1758,7 +1764,7 @@ static int step_impl(lbm_solver* s, int nsteps, int* done, std::vector<hipEvent_
       s->pending_what.push_back(2);
       s->pending++;
     }
-    const bool feval = !s->force_pass && forces_at(s->iter);
+    const bool feval = !fpass && forces_at(s->iter);
     // The history is read after a single step: a divergence that it shows ends
     // the call there, with the state one step back in buf[cur^1].
     const bool full = s->pending >= HCAP;
