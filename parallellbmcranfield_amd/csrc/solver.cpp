@@ -448,10 +448,8 @@ static int setup_lds_steps(lbm_solver* s, const std::vector<uint8_t>& cls,
     // The ring of a rectangle holds no node: a lattice's is padding; a packed
     // instance's might (a mesh whose outermost cells are fluid).
     for (int y = r[1]; y < r[3] && s->ninst; y++)
-      for (int x = r[0]; x < r[2]; x++)
-        if ((y == r[1] || y == r[3] - 1 || x == r[0] || x == r[2] - 1) &&
-            cls[(size_t)y * pitch + x] != 0)
-          return LBM_OK;
+      for (int x = r[0]; x < r[2]; x += (y == r[1] || y == r[3] - 1) ? 1 : std::max(1, r[2] - r[0] - 1))
+        if (cls[(size_t)y * pitch + x] != 0) return LBM_OK;
     // the block of output nodes from (x, y), w wide; false where it is left out:
     // no node, or not `plain` where only such a block is asked for
     auto add = [&](int x, int y, int w, bool only_plain) {
