@@ -91,7 +91,8 @@ struct lbm_solver {
   // row of it is zero, and no stop rule reads it: no step evaluates it
   bool ref_zero = false;
   double* d_part = nullptr;   // [nparts][4]
-  double* hist = nullptr;     // [HSLOTS][8] sums of evaluations, pinned: kernels write, the host reads
+  double* hist = nullptr;     // [HSLOTS][8] sums of evaluations, pinned: kernels write, the host reads;
+                              // null where nothing is evaluated
   uint32_t* d_seed = nullptr; // FP16 stochastic rounding: step number, 2 slots
   int nparts = 0;
   int nb_bulk = 0, nb_bnd = 0, nb_out = 0;
@@ -172,7 +173,7 @@ struct lbm_solver {
   uint16_t* d_node_inst = nullptr;
   uint8_t* d_inst_active = nullptr;
   int* d_inst_rect = nullptr;        // storage rectangles [ninst][4]
-  double* inst_raw = nullptr;        // [ninst][2], behind hist
+  double* inst_raw = nullptr;        // [ninst][2]: hist of a packed lattice
   uint32_t* d_tile_list = nullptr;   // bulk tiles of running instances (padded)
   int nb_list = 0;
   std::vector<uint32_t> tile_first;  // tile t's instances: tile_ids[tile_first[t] .. [t+1])
